@@ -159,7 +159,7 @@ int lf_neighbours(lf_scene *s, uint32_t *counts, uint32_t *list, uint64_t cap, u
  * table the normals, forces and XSPH passes walk with the kernels' own code:
  * the non-empty 32-slot pseudo-rows in row order, (entry_mask[k],
  * entry_base[k]) for k < min(*count, 16); *count is the number of non-empty
- * pseudo-rows (above 16 the kernels walk row by row instead).  The entry
+ * pseudo-rows (above 16 the kernels fill and walk a table several times).  The entry
  * arrays hold 16 elements. */
 int lf_debug_flat_table(const uint64_t masks[9], const uint32_t first_slot[9], uint32_t *entry_mask,
                         uint32_t *entry_base, uint32_t *count);
@@ -246,8 +246,7 @@ int lf_export_wait(lf_scene *s);
 int lf_set_tuning(lf_scene *s, const int block_sizes[4]);
 int lf_get_tuning(const lf_scene *s, int block_sizes[4]);
 /* Walk modes of the normals, forces and XSPH passes: 1 walks the density
- * pass's neighbour masks as one flattened stream of set bits (in waves whose
- * stencil rows all fit 64-slot masks), 0 walks them row by row, 2 flattens
+ * pass's neighbour masks as one flattened stream of set bits, 0 walks them row by row, 2 flattens
  * only the waves in which a row holds more than 32 slots.  Default {1, 1, 2}
  * (measured fastest: the force walk's arithmetic-heavy steps gain from the
  * flattened stream everywhere, the XSPH walk's gather-heavy ones only where

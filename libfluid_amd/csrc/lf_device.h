@@ -22,8 +22,9 @@ constexpr uint32_t kScanDirectTiles = 2048;    // above this many tiles the tile
 
 // Neighbour masks of one radius for 9 stencil rows x nslots particle slots,
 // row-major (entry r * nslots + i).  Bit k stands for slot b_r + k of row r.
-// A row of at most 32 slots keeps its mask in w32, a row of 33..64 slots in
-// w64; longer rows have no mask.
+// A row of at most 32 slots keeps its mask in w32, a longer one its first 64
+// slots in w64 and, if it has more than 64, slots 64..95 in w32; the slots
+// from 96 on have no mask (a walk tests them again, fill_long).
 struct RowMasks {
     uint32_t *w32;
     uint64_t *w64;

@@ -64,16 +64,18 @@ void launch_density(const Launch &L, const PoolView &pv, int bs, const float4 *P
 // either way.  launch_normals processes the scenes without lazy_normal,
 // or with `all` every scene (the on-demand normals of the last substep).
 void launch_normals(const Launch &L, const PoolView &pv, int bs, int flat, bool all, const float4 *Q,
-                    const uint32_t *start, RowMasks M, const uint32_t *flags, float4 *N);
+                    const float *soa, const uint32_t *start, RowMasks M, const uint32_t *flags, const uint32_t *moves,
+                    float4 *N);
 // A and Lw are the state arrays, read at order[i]; Aout and Lout must be
 // other buffers (they are written in cell order).
 void launch_forces(const Launch &L, const PoolView &pv, int bs, int flat, const float4 *Ps, const float4 *Q,
                    const float *Pr, const float4 *Vs, const float4 *A, const float4 *Lw, const uint32_t *order,
-                   const float4 *D, const float4 *N, const uint32_t *start, RowMasks M, float4 *Pout, float4 *Vout,
-                   float4 *Aout, float4 *Lout, float4 *Fdbg, uint32_t *flags, const uint32_t *moves);
+                   const float4 *D, const float4 *N, const float *soa, const uint32_t *start, RowMasks M,
+                   float4 *Pout, float4 *Vout, float4 *Aout, float4 *Lout, float4 *Fdbg, uint32_t *flags,
+                   const uint32_t *moves);
 void launch_xsph(const Launch &L, const PoolView &pv, int bs, int flat, const float4 *Ps, const float4 *Pn,
-                 const float4 *Vh, const float4 *Lw, const uint32_t *start, RowMasks MS, const uint32_t *flags,
-                 float4 *Vout);
+                 const float4 *Vh, const float4 *Lw, const float *soa, const uint32_t *start, RowMasks MS,
+                 const uint32_t *flags, const uint32_t *moves, float4 *Vout);
 
 // Per-scene helpers: slots [first, first + count) of one scene.
 void launch_upload(hipStream_t st, const float *stage, uint32_t first, uint32_t id0, uint32_t count, float4 *P,

@@ -22,8 +22,8 @@
 //
 // The density pass tests every candidate of the clipped 27-cell stencil (nine
 // contiguous x-row slot ranges) and records, per row, a 32/64-bit mask of the
-// slots within a skin radius h_s >= h.  The normals, forces and XSPH passes
-// walk those masks over packed neighbour data (XSPH when the substep's
+// slots within a skin radius h_s >= h (of its first 96 slots; RowMasks).
+// The normals, forces and XSPH passes walk those masks over packed neighbour data (XSPH when the substep's
 // largest move proves them complete) and re-test each pair; set bits are
 // visited in slot order, so every pass sums the same neighbours in the same
 // order as a full stencil scan, bit for bit.
@@ -457,8 +457,8 @@ __device__ __forceinline__ void rows9(const Consts &c, const uint32_t *__restric
 // skin radius (bit k = slot b[r] + k), a superset of the neighbours within h,
 // which the callbacks re-test.  walk_masks visits the set bits in increasing
 // slot order, the
-// same order as a full scan; a row longer than 64 slots has no mask and is
-// scanned in full.  With use == false every row is scanned.  Each step takes
+// same order as a full scan; a row longer than 64 slots is scanned in full
+// (walk_flat does better).  With use == false every row is scanned.  Each step takes
 // up to W set bits of the row and issues all their candidates' loads (ld)
 // before using them (fn, in slot order), so W gathers per lane are in flight
 // at a time.  fn(cand, slot, ok) adds nothing when ok is false (a step with
@@ -550,60 +550,161 @@ __device__ __forceinline__ void walk_masks(const uint32_t *b, const uint32_t *e,
     }
 }
 
-// Flattened walk of the nine rows' masks.  Iterating row by row costs every
-// row the longest run of any lane in the wave; one stream of set bits over
-// all rows costs only the largest total.  Each lane splits its rows into
-// pseudo-rows of at most 32 slots (a row of 33..64 slots is two: its 64-bit
-// mask's low and high words, the second starting 32 slots later), compacts
-// the non-empty ones, (mask, first slot), into its own column of the
-// workgroup's LDS table tab[kFlatEntries][BS] and walks them in row order,
-// W set bits per step (consecutive bits may come from adjacent pseudo-rows):
-// the W candidates' loads are all issued before the first is used, so W
-// gathers per lane are in flight.  The next entry is fetched one entry
-// ahead, so a row change does not wait on LDS.  Visits the same slots in the
-// same order as walk_masks.  Returns false, having visited nothing, when a
-// lane of the wave has a row of more than 64 slots or more than kFlatEntries
-// non-empty pseudo-rows, or (need_long) when no lane of the wave has a row
-// of more than 32 slots (one pseudo-row per row: the row-by-row walk then
-// does as well without the table).  The table is filled by flat_table.
-constexpr int kForceWalkWidth = 4;  // set bits per step of the flattened force walk
-constexpr int kXsphWalkWidth = 4;   // and of the flattened XSPH walk
-constexpr int kXsphRowWidth = 4;    // set bits per step of the row-by-row XSPH walk
-template <int BS, int W, class Ld, class Fn>
-__device__ __forceinline__ bool walk_flat(uint2 *__restrict__ tab, const uint32_t *b, const uint32_t *e,
-                                          const RowMasks &mask, uint32_t nslots, uint32_t i, bool need_long, Ld &&ld,
-                                          Fn &&fn) {
+// Row r (wave-uniform) of the particle at pc: its first slot and its end,
+// as rows9 gives them.
+__device__ __forceinline__ uint2 row_span(const Consts &c, const uint32_t *__restrict__ start, uint32_t shift,
+                                          float4 pc, uint32_t r) {
+    int cx, cy, cz;
+    cell_xyz(c, pc, cx, cy, cz);
+    const int x0 = cx > 0 ? cx - 1 : 0, x1 = cx < c.gx - 1 ? cx + 1 : c.gx - 1;
+    const int z = cz + (int)(r / 3u) - 1, y = cy + (int)(r % 3u) - 1;
+    const bool ok = z >= 0 && z < c.gz && y >= 0 && y < c.gy;
+    const uint32_t row = (uint32_t)((ok ? z : cz) * c.gy + (ok ? y : cy)) * (uint32_t)c.gx;
+    const uint32_t bb = start[row + (uint32_t)x0] + shift;
+    const uint32_t ee = start[row + (uint32_t)x1 + 1u] + shift;
+    return make_uint2(bb, ok ? ee : bb);
+}
+
+// Long rows.  What the walks need to find a row's mask words without the
+// row table in registers: the scene, its cell table, the pre-integration
+// positions (also as planes) and the largest move, which gives the skin
+// radius of the density pass; and, for XSPH in a scene whose masks are not
+// complete, the integrated positions to test instead (moved; null elsewhere).
+struct RowSource {
+    const Consts &c;
+    const uint32_t *__restrict__ st;
+    uint32_t shift;
+    const float4 *__restrict__ pos;  // pre-integration positions, cell order
+    const float *__restrict__ soa;
+    const uint32_t *__restrict__ moves;
+    const float4 *__restrict__ moved;
+};
+
+// Mask word of up to 32 slots [s, s + n) (n of them, at most 32 used),
+// tested against the skin radius exactly as the density pass tests them.
+__device__ __forceinline__ uint32_t skin_word(const RowSource &src, uint32_t nslots, float4 pc, uint32_t s,
+                                              uint32_t n, uint32_t i) {
+    const __amdgpu_buffer_rsrc_t px = plane_buffer(src.soa, nslots), py = plane_buffer(src.soa + nslots, nslots),
+                                 pz = plane_buffer(src.soa + 2 * (size_t)nslots, nslots);
+    const float nh2s = -skin_h2s(src.c, skin_frac(scene_move_q(src.moves, src.c.scene)));
+    const uint32_t off = s * (uint32_t)sizeof(float);
+    uint32_t cur = 0u;
+    auto test = [&](float qx, float qy, float qz) {
+        const float dx = qx - pc.x, dy = qy - pc.y, dz = qz - pc.z;
+        const float rs = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, nh2s)));
+        cur = __builtin_amdgcn_alignbit(cur, __float_as_uint(rs), 31u);
+    };
+#pragma unroll 1
+    for (uint32_t so = 0u; so < 32u * (uint32_t)sizeof(float); so += 4u * (uint32_t)sizeof(float)) {
+        const float4 X = load4(px, off, so), Y = load4(py, off, so), Z = load4(pz, off, so);
+        test(X.x, Y.x, Z.x);
+        test(X.y, Y.y, Z.y);
+        test(X.z, Y.z, Z.z);
+        test(X.w, Y.w, Z.w);
+    }
+    uint32_t m = __brev(cur);
+    if (n < 32u) m &= (1u << n) - 1u;
+    const uint32_t k = i - s;  // the particle itself is no candidate
+    if (k < 32u) m &= ~(1u << k);
+    return m;
+}
+
+// Mask word of up to 32 slots [s, s + n) by the integrated positions: those
+// within h (the pair test of the XSPH walk itself).
+__device__ __forceinline__ uint32_t moved_word(const RowSource &src, uint32_t s, uint32_t n, uint32_t i) {
+    uint32_t cur = 0u;
+    if (n > 32u) n = 32u;
+    const float4 xi = at32(src.moved, i);
+#pragma unroll 1
+    for (uint32_t g = 0u; g < n; g += 4u) {
+        float4 q[4];
+#pragma unroll
+        for (uint32_t k = 0u; k < 4u; ++k) q[k] = at32(src.moved, g + k < n ? s + g + k : s);
+#pragma unroll
+        for (uint32_t k = 0u; k < 4u; ++k)
+            cur |= g + k < n && dist2(xi, q[k]) <= src.c.h2 ? 1u << (g + k) : 0u;
+    }
+    const uint32_t k = i - s;  // the particle itself is no candidate
+    if (k < 32u) cur &= ~(1u << k);
+    return cur;
+}
+
+// The stored mask of a row's first 64 slots by one unconditional 8-byte load:
+// from the 64-bit array for a row of more than 32 slots, else from the 32-bit
+// array, whose allocation is padded so that the word after the last entry is
+// readable (that second word is dropped).
+__device__ __forceinline__ uint64_t row_mask64(const RowMasks &mask, size_t at, uint32_t len) {
+    const char *p = len > 32u ? reinterpret_cast<const char *>(mask.w64 + at)
+                              : reinterpret_cast<const char *>(mask.w32 + at);
+    uint64_t v;
+    __builtin_memcpy(&v, p, sizeof(v));
+    return len > 32u ? v : (v & 0xFFFFFFFFull);
+}
+
+// Fills the lane's column of the flattened walk's table with its next
+// pseudo-rows, from word `word` of row `row` on (both wave-uniform, left at
+// the first pseudo-row that did not fit), and returns how many it stored.
+// The first three words of a row come from the density pass's masks; later
+// ones (rows of more than 96 slots) are tested again here, 7 VALU
+// instructions a candidate against the 25 to 60 of the walk it spares.  Row
+// bounds and words are loaded anew for each batch, two rows and one row
+// ahead of their use, instead of being held in registers through the walk.
+// With src.moved every word is tested on the integrated positions.
+template <int BS>
+__device__ __forceinline__ uint32_t fill_long(uint2 *__restrict__ tab, const RowSource &src, const RowMasks &mask,
+                                              uint32_t nslots, uint32_t i, uint32_t &row, uint32_t &word) {
     const uint32_t t = threadIdx.x;
-    if (need_long) {
-        bool lng = false;
-#pragma unroll
-        for (int r = 0; r < 9; ++r) lng = lng || e[r] - b[r] > 32u;
-        if (!__ballot(lng)) return false;
+    struct Span {
+        uint32_t s, len;
+    };
+    struct Words {
+        uint64_t w01;
+        uint32_t w2;
+    };
+    const float4 pc = at32(src.pos, i);
+    const auto span = [&](uint32_t r) {
+        const uint2 x = row_span(src.c, src.st, src.shift, pc, r < 9u ? r : 8u);
+        return Span{x.x, x.y - x.x};
+    };
+    const auto words = [&](uint32_t r, uint32_t len) {
+        const size_t at = (size_t)(r < 9u ? r : 8u) * nslots + i;
+        return Words{row_mask64(mask, at, len), mask.w32[at]};  // w2: slots 64..95 of a row of more than 64
+    };
+    Span cur = span(row), nxt = span(row + 1u);
+    Words w = words(row, cur.len);
+    uint32_t cnt = 0u, used = 0u;
+#pragma unroll 1
+    while (row < 9u) {
+        const Words wn = words(row + 1u, nxt.len);
+        const Span nn = span(row + 2u);
+#pragma unroll 1
+        for (; __ballot(cur.len > 32u * word); ++word) {
+            if (used == (uint32_t)kFlatEntries) return cnt;
+            const bool in = cur.len > 32u * word;
+            uint32_t m = word == 0u ? (uint32_t)w.w01 : word == 1u ? (uint32_t)(w.w01 >> 32) : w.w2;
+            if (src.moved)
+                m = in ? moved_word(src, cur.s + 32u * word, cur.len - 32u * word, i) : 0u;
+            else if (word >= 3u)
+                m = in ? skin_word(src, nslots, pc, cur.s + 32u * word, cur.len - 32u * word, i) : 0u;
+            if (in && m != 0u) {
+                tab[cnt * BS + t] = make_uint2(m, cur.s + 32u * word);
+                ++cnt;
+            }
+            ++used;
+        }
+        word = 0u;
+        ++row;
+        cur = nxt;
+        w = wn;
+        nxt = nn;
     }
-    // Each row's mask with one unconditional 8-byte load (from the 64-bit
-    // array for a row of 33..64 slots, else from the 32-bit array, whose
-    // allocation is padded so that the word after the last entry is
-    // readable; that second word is then dropped), so the nine loads are in
-    // flight together.
-    uint64_t mw[9];
-    bool fits = true;
-#pragma unroll
-    for (int r = 0; r < 9; ++r) {
-        const uint32_t len = e[r] - b[r];
-        const size_t at = (size_t)r * nslots + i;
-        const char *src = len > 32u ? reinterpret_cast<const char *>(mask.w64 + at)
-                                    : reinterpret_cast<const char *>(mask.w32 + at);
-        uint64_t v;
-        __builtin_memcpy(&v, src, sizeof(v));
-        mw[r] = len > 32u ? v : (v & 0xFFFFFFFFull);
-        fits = fits && len <= 64u;
-    }
-    // Entries at or past cnt are never stored and never used (the reads
-    // below that may touch them are discarded).
-    const uint32_t cnt = flat_table(mw, b, [&](uint32_t k, uint32_t m, uint32_t base) {
-        tab[k * BS + t] = make_uint2(m, base);
-    });
-    if (__ballot(!fits || cnt > (uint32_t)kFlatEntries)) return false;
+    return cnt;
+}
+
+// Visits the set bits of the lane's first cnt table entries, W per step.
+template <int BS, int W, class Ld, class Fn>
+__device__ __forceinline__ void walk_table(const uint2 *__restrict__ tab, uint32_t cnt, Ld &&ld, Fn &&fn) {
+    const uint32_t t = threadIdx.x;
     const uint2 e0 = tab[t];
     uint32_t m = cnt > 0u ? e0.x : 0u, base = e0.y;
     uint2 nx = tab[BS + t];  // entry nxt as read: used only if nxt < cnt
@@ -638,7 +739,88 @@ __device__ __forceinline__ bool walk_flat(uint2 *__restrict__ tab, const uint32_
 #pragma unroll
         for (int k = 0; k < W; ++k) fn(a[k], j[k], ok[k]);
     }
-    return true;
+}
+
+// Flattened walk of the nine rows' masks.  Iterating row by row costs every
+// row the longest run of any lane in the wave; one stream of set bits over
+// all rows costs only the largest total.  Each lane splits its rows into
+// pseudo-rows of at most 32 slots (a row of 33..64 slots is two: its 64-bit
+// mask's low and high words, the second starting 32 slots later), compacts
+// the non-empty ones, (mask, first slot), into its own column of the
+// workgroup's LDS table tab[kFlatEntries][BS] and walks them in row order,
+// W set bits per step (consecutive bits may come from adjacent pseudo-rows):
+// the W candidates' loads are all issued before the first is used, so W
+// gathers per lane are in flight.  The next entry is fetched one entry
+// ahead, so a row change does not wait on LDS.  Visits the same slots in the
+// same order as walk_masks.
+//
+// A wave in which a lane has a row of more than 64 slots, or more than
+// kFlatEntries non-empty pseudo-rows, fills and walks its table several times
+// (fill_long).  Such rows are everyday in the default double dam break (h is
+// 2.3 particle spacings there: rows of up to 81 slots at rest density) and in
+// compressed fluid; while their waves scanned those rows slot by slot, one
+// dependent load each, normals / forces / XSPH of the 200,000-particle double
+// dam with every force term took 172 / 366 / 175 us late in the splash and
+// 91 / 178 / 106 early, against 73 / 203 / 158 and 39 / 127 / 55 this way;
+// rows of 192 slots (100,000 particles at h/4): forces and XSPH 371 / 308 us
+// against 167 / 143.  Near-isolated waves (WL = 0) keep the slot-by-slot
+// scan: they hardly ever have such rows, and the batches would cost their
+// walk registers.  Returns false, having visited nothing, in that case and
+// when (need_long) no lane of the wave has a row of more than 32 slots (one
+// pseudo-row per row: the row-by-row walk then does as well without the
+// table).  The table is filled by flat_table.
+constexpr int kForceWalkWidth = 4;  // set bits per step of the flattened force walk
+constexpr int kForceLongWidth = 3;  // and where a wave's rows need more than one table
+constexpr int kXsphWalkWidth = 4;   // and of the flattened XSPH walk
+constexpr int kXsphRowWidth = 4;    // set bits per step of the row-by-row XSPH walk
+template <int BS, int W, int WL, class Ld, class Fn>
+__device__ __forceinline__ bool walk_flat(uint2 *__restrict__ tab, const RowSource &src, const uint32_t *b,
+                                          const uint32_t *e, const RowMasks &mask, uint32_t nslots, uint32_t i,
+                                          bool need_long, Ld &&ld, Fn &&fn) {
+    const uint32_t t = threadIdx.x;
+    bool batches = src.moved != nullptr;
+    uint32_t cnt = 0u;
+    if (__builtin_expect(!batches, 1)) {
+        if (need_long) {
+            bool lng = false;
+#pragma unroll
+            for (int r = 0; r < 9; ++r) lng = lng || e[r] - b[r] > 32u;
+            if (!__ballot(lng)) return false;
+        }
+        // The nine masks' loads (row_mask64) are unconditional, so that all
+        // are in flight together.
+        uint64_t mw[9];
+        bool fits = true;
+#pragma unroll
+        for (int r = 0; r < 9; ++r) {
+            const uint32_t len = e[r] - b[r];
+            mw[r] = row_mask64(mask, (size_t)r * nslots + i, len);
+            fits = fits && len <= 64u;
+        }
+        // Entries at or past cnt are never stored and never used (the reads
+        // in walk_table that may touch them are discarded).
+        cnt = flat_table(mw, b, [&](uint32_t k, uint32_t m, uint32_t base) {
+            tab[k * BS + t] = make_uint2(m, base);
+        });
+        batches = __ballot(!fits || cnt > (uint32_t)kFlatEntries) != 0ull;
+    }
+    if (__builtin_expect(!batches, 1)) {
+        walk_table<BS, W>(tab, cnt, ld, fn);
+        return true;
+    }
+    // Rows without a 64-bit mask, or more pseudo-rows than entries, in some
+    // lane: the wave walks batch after batch of its pseudo-rows.  (WL set
+    // bits per step: the force walk takes one fewer here, the fill's state
+    // would otherwise cost every scene's force pass a wave per SIMD.)
+    if constexpr (WL != 0) {
+        uint32_t row = 0u, word = 0u;  // of the next pseudo-row (wave-uniform)
+#pragma unroll 1
+        while (row < 9u) {
+            cnt = fill_long<BS>(tab, src, mask, nslots, i, row, word);
+            walk_table<BS, WL>(tab, cnt, ld, fn);
+        }
+    }
+    return WL != 0;
 }
 
 // Walk over the neighbour slots of lane i: with flat set, the flattened walk
@@ -648,12 +830,12 @@ __device__ __forceinline__ bool walk_flat(uint2 *__restrict__ tab, const uint32_
 // multiply-add contraction may differ between those copies: the callbacks
 // write their multiply-adds as explicit fmaf, so every copy computes the
 // same bits.
-template <int BS, int W, int WR, bool PAIR = false, class Ld, class Fn>
-__device__ __forceinline__ void walk_rows(uint2 *__restrict__ tab, const uint32_t *b, const uint32_t *e,
-                                          const RowMasks &mask, bool use, int flat, uint32_t nslots, uint32_t i,
-                                          Ld &&ld, Fn &&fn) {
-    if (use && flat && walk_flat<BS, W>(tab, b, e, mask, nslots, i, flat == 2, ld, fn)) return;
-    walk_masks<WR, PAIR>(b, e, mask, use, nslots, i, ld, fn);
+template <int BS, int W, int WL, int WR, bool PAIR = false, class Ld, class Fn>
+__device__ __forceinline__ void walk_rows(uint2 *__restrict__ tab, const RowSource &src, const uint32_t *b,
+                                          const uint32_t *e, const RowMasks &mask, bool use, int flat,
+                                          uint32_t nslots, uint32_t i, Ld &&ld, Fn &&fn) {
+    if (use && flat && walk_flat<BS, W, WL>(tab, src, b, e, mask, nslots, i, flat == 2, ld, fn)) return;
+    walk_masks<WR, PAIR>(b, e, mask, use && !src.moved, nslots, i, ld, fn);
 }
 
 // 5. density + Tait EOS (computeDensity, fluidphysics.cu:8-84); also the
@@ -772,20 +954,22 @@ __global__ __launch_bounds__(BS) void k_density(const Consts *__restrict__ cs, c
             s1 = cur;
         else
             s0 = cur;
-        for (k = 64u; k < len; ++k) {  // rows of more than 64 slots: no masks
-            const float4 q = at32(Ps, bb + k);
-            const float dx = q.x - pi.x, dy = q.y - pi.y, dz = q.z - pi.z;
-            const float rs = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, nh2s)));
-            const float t = fminf(fmaxf(__builtin_fmaf(rs, ninv_h2, c1), 0.0f), 1.0f);
-            const float tk = (r != 4 || k != kself) ? t : 0.0f;
-            S = __builtin_fmaf(tk * tk, tk, S);
-        }
         const size_t at = (size_t)r * nslots + i;
         s0 = n0 ? __brev(s0) >> (32u - n0) : 0u;  // n0 == 0: nothing scanned
-        if (len <= 32u) {
+        if (len <= 32u)
             MS.w32[at] = s0;
-        } else if (len <= 64u) {
-            MS.w64[at] = (uint64_t)(__brev(s1) >> (64u - lw)) << 32 | s0;  // lw >= len > 32
+        else
+            MS.w64[at] = (uint64_t)(__brev(s1) >> (64u - lw)) << 32 | s0;  // lw > 32
+        // A row's slots past 64, a mask word at a time (the first is kept).
+        // (One group per step: two cost a wave per SIMD of every scene.)
+        for (uint32_t k0 = 64u; k0 < len; k0 += 32u) {
+            const uint32_t end = k0 + 32u < len ? k0 + 32u : len;
+            cur = 0u;
+            for (k = k0; k < end; k += 4u) {
+                const uint32_t vo = off + k * (uint32_t)sizeof(float);
+                group.template operator()<false>(load4(px, vo, 0u), load4(py, vo, 0u), load4(pz, vo, 0u), k);
+            }
+            if (k0 == 64u) MS.w32[at] = __brev(cur) >> (32u - (k - k0));
         }
     }
     if (S < c.fragile_S) {
@@ -873,8 +1057,9 @@ __device__ __forceinline__ void normal_term(const Consts &c, float4 pi, float4 q
 template <int BS>
 __global__ __launch_bounds__(BS) void k_normals(const Consts *__restrict__ cs, const uint32_t *__restrict__ chunk,
                                                 uint32_t nslots, const float4 *__restrict__ Q,
-                                                const uint32_t *__restrict__ start, RowMasks M, int flat, int all,
-                                                const uint32_t *__restrict__ flags,
+                                                const float *__restrict__ soa, const uint32_t *__restrict__ start,
+                                                RowMasks M, int flat, int all, const uint32_t *__restrict__ flags,
+                                                const uint32_t *__restrict__ moves,
                                                 const uint8_t *__restrict__ near, float4 *__restrict__ N) {
     uint32_t slot0;
     const Consts *cp = block_scene<BS>(cs, chunk, slot0);
@@ -891,11 +1076,12 @@ __global__ __launch_bounds__(BS) void k_normals(const Consts *__restrict__ cs, c
     const float4 pi = Q[i];
     uint32_t b[9], e[9];
     rows9(c, st, shift, pi, b, e);
+    const RowSource rows{c, st, shift, Q, soa, moves, nullptr};
     float sx = 0.0f, sy = 0.0f, sz = 0.0f;
     __shared__ uint2 tab[kFlatEntries * BS];
     auto walk = [&]<bool F>() {
-        walk_rows<BS, 2, 2>(
-            tab, b, e, M, c.use_masks, flat, nslots, i, [&](uint32_t j) { return at32(Q, j); },
+        walk_rows<BS, 2, F ? 0 : 2, 2>(
+            tab, rows, b, e, M, c.use_masks, flat, nslots, i, [&](uint32_t j) { return at32(Q, j); },
             [&](const float4 &q, uint32_t, bool ok) { normal_term<F>(c, pi, q, dist2(pi, q), ok, sx, sy, sz); });
     };
     if (__builtin_expect(flag_set(flag_word(flags, c.scene), kFragileByte), 0) && lanes(rows_near(near, b, e)))
@@ -919,7 +1105,8 @@ __global__ __launch_bounds__(BS) void k_forces(const Consts *__restrict__ cs, co
                                                const float4 *__restrict__ Vs, const float4 *__restrict__ A,
                                                const float4 *__restrict__ Lw, const uint32_t *__restrict__ order,
                                                const float4 *__restrict__ D,
-                                               const float4 *__restrict__ N, const uint32_t *__restrict__ start,
+                                               const float4 *__restrict__ N, const float *__restrict__ soa,
+                                               const uint32_t *__restrict__ start,
                                                RowMasks M, int flat, float4 *__restrict__ Pout,
                                                float4 *__restrict__ Vout, float4 *__restrict__ Aout,
                                                float4 *__restrict__ Lout,
@@ -950,6 +1137,7 @@ __global__ __launch_bounds__(BS) void k_forces(const Consts *__restrict__ cs, co
         float Tx = 0.f, Ty = 0.f, Tz = 0.f;  // cohesion + curvature sum
         uint32_t b[9], e[9];
         rows9(c, st, shift, pi, b, e);
+        const RowSource rows{c, st, shift, Ps, soa, moves, nullptr};
         // One walk per combination of the scene's optional terms, so that a
         // candidate's loads (V: velocity and density/sound speed; T: normal)
         // are all issued with its position before any arithmetic.  F: the
@@ -968,8 +1156,8 @@ __global__ __launch_bounds__(BS) void k_forces(const Consts *__restrict__ cs, co
             };
             // (two set bits per step in the near-isolated walk: its FP64
             // terms would otherwise cost every scene's walk registers)
-            walk_rows<BS, F ? 2 : kForceWalkWidth, 2>(
-                tab, b, e, M, c.use_masks, flat, nslots, i,
+            walk_rows<BS, F ? 2 : kForceWalkWidth, F ? 0 : kForceLongWidth, 2>(
+                tab, rows, b, e, M, c.use_masks, flat, nslots, i,
                 [&](uint32_t j) {
                     Cand cd;
                     cd.q = at32(Q, j);
@@ -1161,16 +1349,19 @@ __global__ __launch_bounds__(BS) void k_forces(const Consts *__restrict__ cs, co
 // a pair within h after the move was within h + 2 max|dx| before it, so the
 // masks are complete while no particle moved farther than move_limit
 // (h + 2 move_limit <= h_s with FP32 margins); k_forces flags a farther move
-// in the scene's far-move flag, and then every row is scanned.  Registers
+// in the scene's far-move flag, and then every row's slots are tested again
+// on the integrated positions (moved_word; the default driver's splash, 87
+// against 106 us for 10,000 particles scanned).  Registers
 // are capped for five waves per SIMD (four for 512-thread workgroups).
 template <int BS>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(BS >= 512 ? 4 : 5))) void k_xsph(
                                              const Consts *__restrict__ cs, const uint32_t *__restrict__ chunk,
                                              uint32_t nslots, const float4 *__restrict__ Ps,
                                              const float4 *__restrict__ Pn, const float4 *__restrict__ Vh,
-                                             const float4 *__restrict__ Lw, const uint32_t *__restrict__ start,
+                                             const float4 *__restrict__ Lw, const float *__restrict__ soa,
+                                             const uint32_t *__restrict__ start,
                                              RowMasks MS, int flat, const uint32_t *__restrict__ flags,
-                                             const uint8_t *__restrict__ near,
+                                             const uint32_t *__restrict__ moves, const uint8_t *__restrict__ near,
                                              float4 *__restrict__ Vout) {
     uint32_t slot0;
     const Consts *cp = block_scene<BS>(cs, chunk, slot0);
@@ -1186,10 +1377,11 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(BS >= 512 ? 
         return;
     }
     const uint32_t fl = flag_word(flags, c.scene);
-    const bool masks_ok = c.use_masks && !flag_set(fl, kFarMoveByte);
     const float4 xi = Pn[i];
     const float rho_i = vi.w;
     uint32_t b[9], e[9];
+    // a particle moved farther than the masks allow: test the moved positions
+    const RowSource rows{c, st, shift, Ps, soa, moves, flag_set(fl, kFarMoveByte) ? Pn : nullptr};
     rows9(c, st, shift, Ps[i], b, e);
     float sx = 0.f, sy = 0.f, sz = 0.f;
     const float h2 = c.h2, eps = c.eps;
@@ -1202,8 +1394,8 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(BS >= 512 ? 
     };
     __shared__ uint2 tab[kFlatEntries * BS];
     auto walk = [&]<bool F>() {
-        walk_rows<BS, F ? 2 : kXsphWalkWidth, F ? 2 : kXsphRowWidth, !F>(
-            tab, b, e, MS, masks_ok, flat, nslots, i,
+        walk_rows<BS, F ? 2 : kXsphWalkWidth, F ? 0 : kXsphWalkWidth, F ? 2 : kXsphRowWidth, !F>(
+            tab, rows, b, e, MS, c.use_masks, flat, nslots, i,
             [&](uint32_t j) { return Cand{at32(Pn, j), at32(Vh, j)}; },
             [&](const Cand &cj, uint32_t j, bool ok) {
                 const float4 q = cj.x;
@@ -1531,29 +1723,31 @@ void launch_density(const Launch &L, const PoolView &pv, int bs, const float4 *P
 }
 
 void launch_normals(const Launch &L, const PoolView &pv, int bs, int flat, bool all, const float4 *Q,
-                    const uint32_t *start, RowMasks M, const uint32_t *flags, float4 *N) {
+                    const float *soa, const uint32_t *start, RowMasks M, const uint32_t *flags, const uint32_t *moves,
+                    float4 *N) {
     with_bs(bs, [&]<int BS>() {
-        LF_GO(L, k_normals<BS>, pv.nlaunch / BS, BS, L.a, L.b, pv.cs, pv.chunk, pv.nslots, Q, start, M, flat,
-              all ? 1 : 0, flags, pv.near, N);
+        LF_GO(L, k_normals<BS>, pv.nlaunch / BS, BS, L.a, L.b, pv.cs, pv.chunk, pv.nslots, Q, soa, start, M,
+              flat, all ? 1 : 0, flags, moves, pv.near, N);
     });
 }
 
 void launch_forces(const Launch &L, const PoolView &pv, int bs, int flat, const float4 *Ps, const float4 *Q,
                    const float *Pr, const float4 *Vs, const float4 *A, const float4 *Lw, const uint32_t *order,
-                   const float4 *D, const float4 *N, const uint32_t *start, RowMasks M, float4 *Pout, float4 *Vout,
-                   float4 *Aout, float4 *Lout, float4 *Fdbg, uint32_t *flags, const uint32_t *moves) {
+                   const float4 *D, const float4 *N, const float *soa, const uint32_t *start, RowMasks M,
+                   float4 *Pout, float4 *Vout, float4 *Aout, float4 *Lout, float4 *Fdbg, uint32_t *flags,
+                   const uint32_t *moves) {
     with_bs(bs, [&]<int BS>() {
         LF_GO(L, k_forces<BS>, pv.nlaunch / BS, BS, L.a, L.b, pv.cs, pv.chunk, pv.nslots, Ps, Q, Pr, Vs, A, Lw, order,
-              D, N, start, M, flat, Pout, Vout, Aout, Lout, Fdbg, flags, moves, pv.near);
+              D, N, soa, start, M, flat, Pout, Vout, Aout, Lout, Fdbg, flags, moves, pv.near);
     });
 }
 
 void launch_xsph(const Launch &L, const PoolView &pv, int bs, int flat, const float4 *Ps, const float4 *Pn,
-                 const float4 *Vh, const float4 *Lw, const uint32_t *start, RowMasks MS, const uint32_t *flags,
-                 float4 *Vout) {
+                 const float4 *Vh, const float4 *Lw, const float *soa, const uint32_t *start, RowMasks MS,
+                 const uint32_t *flags, const uint32_t *moves, float4 *Vout) {
     with_bs(bs, [&]<int BS>() {
-        LF_GO(L, k_xsph<BS>, pv.nlaunch / BS, BS, L.a, L.b, pv.cs, pv.chunk, pv.nslots, Ps, Pn, Vh, Lw, start, MS,
-              flat, flags, pv.near, Vout);
+        LF_GO(L, k_xsph<BS>, pv.nlaunch / BS, BS, L.a, L.b, pv.cs, pv.chunk, pv.nslots, Ps, Pn, Vh, Lw, soa,
+              start, MS, flat, flags, moves, pv.near, Vout);
     });
 }
 

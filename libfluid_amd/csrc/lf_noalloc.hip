@@ -210,10 +210,10 @@ extern "C" int lf_step_noalloc(const lf_params *p, uint32_t num_particles, float
         launch_gather(L, pv, b.slot_src, b.slot_id, b.keys, b.start, b.P0, b.V0, b.P1, b.V1, b.ranks, b.soa, b.moves);
         launch_density(L, pv, t.density, b.P1, b.soa, b.start, b.D, b.Q, b.Pr, b.MS, b.flags, b.moves);
         if (!c.lazy_normal)
-            launch_normals(L, pv, t.normals, t.flat_normals, false, b.Q, b.start, b.MS, b.flags, b.N);
-        launch_forces(L, pv, t.forces, t.flat_forces, b.P1, b.Q, b.Pr, b.V1, b.A0, b.L0, b.ranks, b.D, b.N, b.start,
-                      b.MS, b.P0, b.V2, b.A1, b.L1, nullptr, b.flags, b.moves);
-        launch_xsph(L, pv, t.xsph, t.flat_xsph, b.P1, b.P0, b.V2, b.L1, b.start, b.MS, b.flags, b.V0);
+            launch_normals(L, pv, t.normals, t.flat_normals, false, b.Q, b.soa, b.start, b.MS, b.flags, b.moves, b.N);
+        launch_forces(L, pv, t.forces, t.flat_forces, b.P1, b.Q, b.Pr, b.V1, b.A0, b.L0, b.ranks, b.D, b.N, b.soa,
+                      b.start, b.MS, b.P0, b.V2, b.A1, b.L1, nullptr, b.flags, b.moves);
+        launch_xsph(L, pv, t.xsph, t.flat_xsph, b.P1, b.P0, b.V2, b.L1, b.soa, b.start, b.MS, b.flags, b.moves, b.V0);
         std::swap(b.A0, b.A1);
         std::swap(b.L0, b.L1);
     }

@@ -563,14 +563,14 @@ void Pool::enqueue_substep() {
     });
     if (any_separate_normals())
         timed(LF_K_NORMALS, [&](const Launch &L) {
-            launch_normals(L, pv, tune_.normals, tune_.flat_normals, false, Q_, start_, MS_, flags_, N_);
+            launch_normals(L, pv, tune_.normals, tune_.flat_normals, false, Q_, soa_, start_, MS_, flags_, moves_, N_);
         });
     timed(LF_K_FORCES, [&](const Launch &L) {
-        launch_forces(L, pv, tune_.forces, tune_.flat_forces, P1_, Q_, Pr_, V1_, A0_, L0_, ranks_, D_, N_, start_,
-                      MS_, P0_, V2_, A1_, L1_, (debug_ & LF_DEBUG_FORCES) ? F_ : nullptr, flags_, moves_);
+        launch_forces(L, pv, tune_.forces, tune_.flat_forces, P1_, Q_, Pr_, V1_, A0_, L0_, ranks_, D_, N_, soa_,
+                      start_, MS_, P0_, V2_, A1_, L1_, (debug_ & LF_DEBUG_FORCES) ? F_ : nullptr, flags_, moves_);
     });
     timed(LF_K_XSPH, [&](const Launch &L) {
-        launch_xsph(L, pv, tune_.xsph, tune_.flat_xsph, P1_, P0_, V2_, L1_, start_, MS_, flags_, V0_);
+        launch_xsph(L, pv, tune_.xsph, tune_.flat_xsph, P1_, P0_, V2_, L1_, soa_, start_, MS_, flags_, moves_, V0_);
     });
     for (const auto &r : paused_ranges()) launch_carry(stream_, r.first, r.second, A0_, L0_, A1_, L1_);
 }
@@ -804,7 +804,7 @@ int Pool::get_field(uint32_t id, int field, void *dst, size_t bytes) {
                 return fail(LF_ERR_STATE, "normals: no substep data for this scene (none since it was added, "
                                           "loaded, moved, re-parametrised or paused, or autotuning ran since)");
             launch_normals(Launch{stream_, nullptr, nullptr}, view(), tune_.normals, tune_.flat_normals, true,
-                           Q_, start_, MS_, flags_, N_);
+                           Q_, soa_, start_, MS_, flags_, moves_, N_);
             if (int rc = check_launch("normals")) return rc;
             LF_HIP(hipStreamSynchronize(stream_));
             src = N_ + f;
