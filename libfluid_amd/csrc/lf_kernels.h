@@ -28,6 +28,7 @@ struct PoolView {
     uint32_t nslots;
     uint32_t nlaunch;
     uint8_t *near;
+    bool full;  // a scene of the launch has viscosity or surface tension
 };
 
 uint32_t scan_tiles(uint32_t m);

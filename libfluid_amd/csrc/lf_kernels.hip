@@ -838,6 +838,70 @@ __device__ __forceinline__ void walk_rows(uint2 *__restrict__ tab, const RowSour
     walk_masks<WR, PAIR>(b, e, mask, use && !src.moved, nslots, i, ld, fn);
 }
 
+// The near-isolated particle's sum of t^3 over its pairs within h in FP64, in
+// slot order (MS: its own masks, as just stored by this lane).
+__device__ __forceinline__ double near_isolated_sum(const Consts &c, const uint32_t *b, const uint32_t *e,
+                                                    const float4 *__restrict__ Ps, const RowMasks &MS,
+                                                    uint32_t nslots, uint32_t i, float4 pi) {
+    double Sd = 0.0;
+    for (int r = 0; r < 9; ++r) {
+        const uint32_t len = e[r] - b[r];
+        const size_t at = (size_t)r * nslots + i;
+        if (len <= 64u) {
+            // the skin mask: a superset of the pairs within h
+            uint64_t m = len <= 32u ? (uint64_t)MS.w32[at] : MS.w64[at];
+            while (m) {
+                const uint32_t j = b[r] + (uint32_t)__ffsll((unsigned long long)m) - 1u;
+                m &= m - 1ull;
+                const float4 q = at32(Ps, j);
+                if (!(dist2(pi, q) <= c.h2)) continue;
+                const double t = fmax(c.hh_d - dist2_d(pi, q), 0.0);
+                Sd = __builtin_fma(t * t, t, Sd);
+            }
+        } else {
+            for (uint32_t j = b[r]; j < e[r]; ++j) {
+                const float4 q = at32(Ps, j);
+                if (j == i || !(dist2(pi, q) <= c.h2)) continue;
+                const double t = fmax(c.hh_d - dist2_d(pi, q), 0.0);
+                Sd = __builtin_fma(t * t, t, Sd);
+            }
+        }
+    }
+    return Sd;
+}
+
+// What follows the density sum S (sum of m * poly6): the boundary term, the
+// Tait EOS and the particle's packed neighbour data.
+__device__ __forceinline__ void density_finish(const Consts &c, uint32_t i, float4 pi, float S,
+                                               float4 *__restrict__ D, float4 *__restrict__ Q,
+                                               float *__restrict__ Pr, uint32_t *__restrict__ flags,
+                                               uint8_t *__restrict__ near) {
+    // Boundary density term rho0 * (1 - boundaryDensity(d)) for d = |sdf| < h
+    // (fluidphysics.cu:55-61, fluidkernel.cu:45-67), in FP64, written in t = d/h.
+    const double dist = fabs(box_sdf(c, pi.x, pi.y, pi.z));
+    float corrected = S;
+    if (dist < c.h_d) {
+        const double t = dist / c.h_d, t2 = t * t;
+        const double q = 128.0 - 315.0 * t + t * t2 * (420.0 - 378.0 * t2 + t2 * t2 * (180.0 - 35.0 * t2));
+        corrected = (float)((double)S + c.bd_rho0_d * q);
+    }
+    const float rho = (S == 0.0f) ? c.rho0 : corrected;
+    const float ratio = corrected * c.inv_rho0;
+    const float press = (corrected == 0.0f) ? 0.0f : c.eos_scale * (tait_pow(ratio, c.gamma, c.gamma_i) - 1.0f);
+    const float cs_i = c.K * tait_pow(ratio, c.gamma_m1, c.gamma_m1_i);
+    const float ir = 1.0f / rho;
+    // Every pair the later passes treat as near-isolated (1/rho_j or 1/rho_i
+    // above fragile_ir; rho_i + rho_j below fragile_sr, which needs one
+    // density below fragile_sr / 2) has a particle that sets the flag here.
+    if (ir > c.fragile_ir || rho < 0.5f * c.fragile_sr) {
+        set_flag(flags, c.scene, kFragileByte, 1u);
+        near[i / kNearBlock] = 1u;
+    }
+    D[i] = make_float4(rho, press, cs_i, ir);
+    Q[i] = make_float4(pi.x, pi.y, pi.z, rho > c.eps ? ir : -1.0f);
+    Pr[i] = press;
+}
+
 // 5. density + Tait EOS (computeDensity, fluidphysics.cu:8-84); also the
 // neighbour masks of the substep and the packed neighbour data of the later
 // passes: Q = (x, y, z, 1/density, or -1 when density <= FLT_MIN), Pr =
@@ -976,58 +1040,12 @@ __global__ __launch_bounds__(BS) void k_density(const Consts *__restrict__ cs, c
         // Near-isolated: the same pairs again, in the same order, with the
         // pair geometry in FP64 (the FP32 h^2 - r^2 of a pair near r = h
         // carries a large relative error, and here few pairs make the sum).
-        double Sd = 0.0;
-        for (int r = 0; r < 9; ++r) {
-            const uint32_t len = e[r] - b[r];
-            const size_t at = (size_t)r * nslots + i;
-            if (len <= 64u) {
-                // the skin mask: a superset of the pairs within h
-                uint64_t m = len <= 32u ? (uint64_t)MS.w32[at] : MS.w64[at];
-                while (m) {
-                    const uint32_t j = b[r] + (uint32_t)__ffsll((unsigned long long)m) - 1u;
-                    m &= m - 1ull;
-                    const float4 q = at32(Ps, j);
-                    if (!(dist2(pi, q) <= c.h2)) continue;
-                    const double t = fmax(c.hh_d - dist2_d(pi, q), 0.0);
-                    Sd = __builtin_fma(t * t, t, Sd);
-                }
-            } else {
-                for (uint32_t j = b[r]; j < e[r]; ++j) {
-                    const float4 q = at32(Ps, j);
-                    if (j == i || !(dist2(pi, q) <= c.h2)) continue;
-                    const double t = fmax(c.hh_d - dist2_d(pi, q), 0.0);
-                    Sd = __builtin_fma(t * t, t, Sd);
-                }
-            }
-        }
+        const double Sd = near_isolated_sum(c, b, e, Ps, MS, nslots, i, pi);
         S = (float)(Sd * c.mC6_d);
     } else {
         S *= c.mC6h6;  // sum of m * poly6
     }
-    // Boundary density term rho0 * (1 - boundaryDensity(d)) for d = |sdf| < h
-    // (fluidphysics.cu:55-61, fluidkernel.cu:45-67), in FP64, written in t = d/h.
-    const double dist = fabs(box_sdf(c, pi.x, pi.y, pi.z));
-    float corrected = S;
-    if (dist < c.h_d) {
-        const double t = dist / c.h_d, t2 = t * t;
-        const double q = 128.0 - 315.0 * t + t * t2 * (420.0 - 378.0 * t2 + t2 * t2 * (180.0 - 35.0 * t2));
-        corrected = (float)((double)S + c.bd_rho0_d * q);
-    }
-    const float rho = (S == 0.0f) ? c.rho0 : corrected;
-    const float ratio = corrected * c.inv_rho0;
-    const float press = (corrected == 0.0f) ? 0.0f : c.eos_scale * (tait_pow(ratio, c.gamma, c.gamma_i) - 1.0f);
-    const float cs_i = c.K * tait_pow(ratio, c.gamma_m1, c.gamma_m1_i);
-    const float ir = 1.0f / rho;
-    // Every pair the later passes treat as near-isolated (1/rho_j or 1/rho_i
-    // above fragile_ir; rho_i + rho_j below fragile_sr, which needs one
-    // density below fragile_sr / 2) has a particle that sets the flag here.
-    if (ir > c.fragile_ir || rho < 0.5f * c.fragile_sr) {
-        set_flag(flags, c.scene, kFragileByte, 1u);
-        near[i / kNearBlock] = 1u;
-    }
-    D[i] = make_float4(rho, press, cs_i, ir);
-    Q[i] = make_float4(pi.x, pi.y, pi.z, rho > c.eps ? ir : -1.0f);
-    Pr[i] = press;
+    density_finish(c, i, pi, S, D, Q, Pr, flags, near);
 }
 
 // 6. surface normals (computeNormals, fluidphysics.cu:154-210):
@@ -1040,18 +1058,14 @@ __global__ __launch_bounds__(BS) void k_density(const Consts *__restrict__ cs, c
 // F: the scene has near-isolated particles; a pair with one takes h^2 - r^2
 // in FP64.
 template <bool F>
-__device__ __forceinline__ void normal_term(const Consts &c, float4 pi, float4 q, float rr, bool ok, float &sx,
-                                            float &sy, float &sz) {
+__device__ __forceinline__ float normal_weight(const Consts &c, float4 pi, float4 q, float rr, bool ok) {
     float t = fmaxf(c.h2 - rr, 0.0f);
     t = ok && rr > c.eps ? t : 0.0f;
     if constexpr (F) {
         if (t > 0.0f && q.w > c.fragile_ir)  // near-isolated neighbour: FP64 pair geometry
             t = (float)fmax(c.hh_d - dist2_d(pi, q), 0.0);
     }
-    const float w = t * t * fmaxf(q.w, 0.0f);
-    sx = __builtin_fmaf(w, pi.x - q.x, sx);
-    sy = __builtin_fmaf(w, pi.y - q.y, sy);
-    sz = __builtin_fmaf(w, pi.z - q.z, sz);
+    return t * t * fmaxf(q.w, 0.0f);
 }
 
 template <int BS>
@@ -1082,7 +1096,12 @@ __global__ __launch_bounds__(BS) void k_normals(const Consts *__restrict__ cs, c
     auto walk = [&]<bool F>() {
         walk_rows<BS, 2, F ? 0 : 2, 2>(
             tab, rows, b, e, M, c.use_masks, flat, nslots, i, [&](uint32_t j) { return at32(Q, j); },
-            [&](const float4 &q, uint32_t, bool ok) { normal_term<F>(c, pi, q, dist2(pi, q), ok, sx, sy, sz); });
+            [&](const float4 &q, uint32_t, bool ok) {
+                const float w = normal_weight<F>(c, pi, q, dist2(pi, q), ok);
+                sx = __builtin_fmaf(w, pi.x - q.x, sx);
+                sy = __builtin_fmaf(w, pi.y - q.y, sy);
+                sz = __builtin_fmaf(w, pi.z - q.z, sz);
+            });
     };
     if (__builtin_expect(flag_set(flag_word(flags, c.scene), kFragileByte), 0) && lanes(rows_near(near, b, e)))
         walk.template operator()<true>();
@@ -1091,191 +1110,180 @@ __global__ __launch_bounds__(BS) void k_normals(const Consts *__restrict__ cs, c
     N[i] = make_float4(c.hmCg6 * sx, c.hmCg6 * sy, c.hmCg6 * sz, 0.0f);
 }
 
-// 7. forces (computeAllForces, fluidphysics.cu:215-352) fused with the
-// leapfrog integrator and boundary clamp (LeapfrogIntegratorOperator,
-// fluidintegrator.cu:11-70).  Out-of-grid particles get zero forces and are
-// still integrated.  Fdbg (may be null) receives the four force components.
-// The pre-XSPH velocity carries the particle's density in w for the XSPH
-// pass, which reads the integrated positions from Pout.  Sets the scene's
-// far-move flag when a particle moved farther than the XSPH skin masks allow.
-template <int BS>
-__global__ __launch_bounds__(BS) void k_forces(const Consts *__restrict__ cs, const uint32_t *__restrict__ chunk,
-                                               uint32_t nslots, const float4 *__restrict__ Ps,
-                                               const float4 *__restrict__ Q, const float *__restrict__ Pr,
-                                               const float4 *__restrict__ Vs, const float4 *__restrict__ A,
-                                               const float4 *__restrict__ Lw, const uint32_t *__restrict__ order,
-                                               const float4 *__restrict__ D,
-                                               const float4 *__restrict__ N, const float *__restrict__ soa,
-                                               const uint32_t *__restrict__ start,
-                                               RowMasks M, int flat, float4 *__restrict__ Pout,
-                                               float4 *__restrict__ Vout, float4 *__restrict__ Aout,
-                                               float4 *__restrict__ Lout,
-                                               float4 *__restrict__ Fdbg, uint32_t *__restrict__ flags,
-                                               const uint32_t *__restrict__ moves, const uint8_t *__restrict__ near) {
-    uint32_t slot0;
-    const Consts *cp = block_scene<BS>(cs, chunk, slot0);
-    if (!cp) return;
-    const Consts &c = *cp;
-    const uint32_t move_q = scene_move_q(moves, c.scene);
-    const uint32_t i = slot0 + threadIdx.x;
-    if (i >= c.first + c.count) return;
-    const uint32_t *st = start + c.cell_base;
-    const uint32_t shift = c.first - st[0];
-    const uint32_t sw = flag_word(flags, c.scene);
-    const uint32_t src = order[i];  // the particle's slot in the state arrays (A, Lw)
-    const float4 pi = Ps[i], vi = Vs[i];
-    const float4 di = D[i];
-    float3 fP = make_float3(0.f, 0.f, 0.f), fV = fP, fT = fP, fA = fP;
-    double eP[3] = {0.0, 0.0, 0.0};  // pressure sum of near-isolated pairs (FP64)
-    if (i < st[c.ncells] + shift) {
-        const float4 ni = c.has_tension ? N[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-        const float rho_i = di.x, p_i = di.y, cs_i = di.z, iri = di.w;
-        const float iri2 = iri * iri;
-        float Px = 0.f, Py = 0.f, Pz = 0.f;  // pressure sum
-        double Pdx = 0.0, Pdy = 0.0, Pdz = 0.0;  // its near-isolated pairs, in FP64
-        float Qx = 0.f, Qy = 0.f, Qz = 0.f;  // artificial-viscosity part of the viscosity sum
-        float Tx = 0.f, Ty = 0.f, Tz = 0.f;  // cohesion + curvature sum
-        uint32_t b[9], e[9];
-        rows9(c, st, shift, pi, b, e);
-        const RowSource rows{c, st, shift, Ps, soa, moves, nullptr};
-        // One walk per combination of the scene's optional terms, so that a
-        // candidate's loads (V: velocity and density/sound speed; T: normal)
-        // are all issued with its position before any arithmetic.  F: the
-        // scene has near-isolated particles, and a pair with one takes its
-        // h - r in FP64 (a separate walk, so that the other scenes' walks
-        // carry none of its registers' cost).
-        __shared__ uint2 tab[kFlatEntries * BS];
-        const bool fragile_i = iri > c.fragile_ir;
-        auto walk = [&]<bool V, bool T, bool F>() {
-            // (with viscosity the neighbour's pressure comes with its
-            // density record, D.y, instead of a load of its own)
-            struct Cand {
-                float4 q;
-                float p;
-                float4 v, d, n;
-            };
-            // (two set bits per step in the near-isolated walk: its FP64
-            // terms would otherwise cost every scene's walk registers)
-            walk_rows<BS, F ? 2 : kForceWalkWidth, F ? 0 : kForceLongWidth, 2>(
-                tab, rows, b, e, M, c.use_masks, flat, nslots, i,
-                [&](uint32_t j) {
-                    Cand cd;
-                    cd.q = at32(Q, j);
-                    if constexpr (V) {
-                        cd.v = at32(Vs, j);
-                        cd.d = at32(D, j);
-                        cd.p = cd.d.y;
-                    } else {
-                        cd.p = at32(Pr, j);
-                    }
-                    if constexpr (T) cd.n = at32(N, j);
-                    return cd;
-                },
-                [&](const Cand &cj, uint32_t, bool ok) {
-                    const float4 q = cj.q;
-                    const float pj = cj.p;
-                    const float rr = dist2(pi, q);
-                    if (!(ok && rr <= c.h2 && rr > c.eps)) return;
-                    if (!(q.w >= 0.0f)) return;  // neighbour density <= FLT_MIN
-                    const float rx = q.x - pi.x, ry = q.y - pi.y, rz = q.z - pi.z;  // x_j - x_i
-                    const float inv_r = frsq(rr);
-                    const float r = rr * inv_r;
-                    const float irj = q.w;
-                    float hr = fmaxf(c.h - r, 0.0f);
-                    bool frag = false;
-                    double hrd = 0.0;
-                    if constexpr (F) {
-                        if (fragile_i || irj > c.fragile_ir) {
-                            // Near-isolated pair: h - r in FP64, r from the
-                            // FP64 r^2 by one Newton step from the FP32 r
-                            // (relative error squared: ~1e-14).
-                            const double d2 = dist2_d(pi, q), r0 = (double)r;
-                            const double rd = __builtin_fma(__builtin_fma(-r0, r0, d2), (double)(0.5f * inv_r), r0);
-                            hrd = fmax(c.h_d - rd, 0.0);
-                            hr = (float)hrd;
-                            frag = true;
-                        }
-                    }
-                    const float cm = c.mCgs * hr * hr * inv_r;  // m gradSpiky(r) / r
-                    if (frag) {
-                        // and its pressure term in FP64: 1/rho^2 of a density
-                        // near FLT_MIN overflows FP32 (an infinite force).
-                        const double cmd = (double)c.mCgs * hrd * hrd * (double)inv_r;
-                        const double midd = __builtin_fma((double)pj, (double)iri * (double)iri,
-                                                          (double)p_i * ((double)irj * (double)irj));
-                        const double cprd = cmd * midd;
-                        Pdx = __builtin_fma(cprd, (double)rx, Pdx);
-                        Pdy = __builtin_fma(cprd, (double)ry, Pdy);
-                        Pdz = __builtin_fma(cprd, (double)rz, Pdz);
-                    } else {
-                        const float mid = __builtin_fmaf(pj, iri2, p_i * (irj * irj));
-                        const float cpr = cm * mid;
-                        Px = __builtin_fmaf(cpr, rx, Px);
-                        Py = __builtin_fmaf(cpr, ry, Py);
-                        Pz = __builtin_fmaf(cpr, rz, Pz);
-                    }
-                    if constexpr (V) {
-                        // Approaching pairs only (ux < 0); the others add exact zeros.
-                        const float4 vj = cj.v, dj = cj.d;
-                        const float ux =
-                            -__builtin_fmaf(vi.z - vj.z, rz, __builtin_fmaf(vi.y - vj.y, ry, (vi.x - vj.x) * rx));
-                        const float mu = c.h * ux * frcp(rr + c.visc_eps);
-                        const float Pi = -c.nu * (cs_i + dj.z) * mu * frcp(rho_i + dj.x);
-                        const float cv = keep(cm * Pi, lanes(ux < 0.0f));
-                        Qx = __builtin_fmaf(cv, rx, Qx);
-                        Qy = __builtin_fmaf(cv, ry, Qy);
-                        Qz = __builtin_fmaf(cv, rz, Qz);
-                    }
-                    if constexpr (T) {
-                        const float4 nj = cj.n;
-                        const float hr3r3 = hr * hr * hr * r * r * r;
-                        const float coh = (r > c.halfh) ? hr3r3 : 2.0f * hr3r3 - c.coh_off;
-                        const float ch = -c.m2 * coh * inv_r;
-                        Tx += __builtin_fmaf(ch, rx, -c.sigma_m * (ni.x - nj.x));
-                        Ty += __builtin_fmaf(ch, ry, -c.sigma_m * (ni.y - nj.y));
-                        Tz += __builtin_fmaf(ch, rz, -c.sigma_m * (ni.z - nj.z));
-                    }
-                });
-        };
-        const bool tension = c.has_tension != 0;
-        auto terms = [&]<bool F>() {
-            if (c.has_visc) {
-                if (tension)
-                    walk.template operator()<true, true, F>();
-                else
-                    walk.template operator()<true, false, F>();
-            } else {
-                if (tension)
-                    walk.template operator()<false, true, F>();
-                else
-                    walk.template operator()<false, false, F>();
-            }
-        };
-        if (flag_set(sw, kFragileByte) && lanes(rows_near(near, b, e)))
-            terms.template operator()<true>();
-        else
-            terms.template operator()<false>();
-        fP = make_float3(Px, Py, Pz);
-        eP[0] = Pdx;
-        eP[1] = Pdy;
-        eP[2] = Pdz;
-        fV = make_float3(c.nu * (Px + Qx), c.nu * (Py + Qy), c.nu * (Pz + Qz));
-        // 2 rho0 / (rho_i + rho_i) applied once to the summed tension terms.
-        const float ts = c.sigma * c.rho0 * iri;
-        fT = make_float3(ts * Tx, ts * Ty, ts * Tz);
-        if (c.has_adhesion) {
-            // Adhesion toward the walls (fluidphysics.cu:330-350), FP64.
-            const double z = -fmin(box_sdf(c, pi.x, pi.y, pi.z), 0.0) * c.quarter_inv_psize;
-            if (z < 1.0) {
-                double nbv[3];
-                box_normal(c, pi.x, pi.y, pi.z, nbv);
-                const double oz = 1.0 - z;
-                const double s = c.alpha_inv_rho0 * (double)rho_i / (oz * oz * oz);
-                fA = make_float3((float)(s * nbv[0]), (float)(s * nbv[1]), (float)(s * nbv[2]));
-            }
+// ---------------------------------------------------------------------------
+// 7. forces: one pair, the sums of a particle's pairs, what follows them.
+
+struct PairSelf {
+    float4 p, v, d, n;  // position, velocity, density record, normal
+    float iri2;         // 1 / density^2
+};
+
+struct PairCand {
+    float4 q;
+    float p;
+    float4 v, d, n;
+};
+
+// A candidate's loads for a walk of the scene's optional terms (V: velocity
+// and density/sound speed; T: normal).  With viscosity the neighbour's
+// pressure comes with its density record, D.y, instead of a load of its own.
+template <bool V, bool T>
+__device__ __forceinline__ PairCand pair_load(const float4 *__restrict__ Q, const float *__restrict__ Pr,
+                                              const float4 *__restrict__ Vs, const float4 *__restrict__ D,
+                                              const float4 *__restrict__ N, uint32_t j) {
+    PairCand cd;
+    cd.q = at32(Q, j);
+    if constexpr (V) {
+        cd.v = at32(Vs, j);
+        cd.d = at32(D, j);
+        cd.p = cd.d.y;
+    } else {
+        cd.p = at32(Pr, j);
+    }
+    if constexpr (T) cd.n = at32(N, j);
+    return cd;
+}
+
+// One pair's contribution: coefficients of x_j - x_i = (rx, ry, rz) in the
+// pressure sum (cpr; cprd in FP64 when frag) and the artificial-viscosity sum
+// (cv), and the cohesion + curvature vector.
+struct PairTerm {
+    float rx, ry, rz, cpr, cv, tx, ty, tz;
+    double cprd;
+    bool frag;
+};
+
+// False (t unset) for a pair that adds nothing.
+template <bool V, bool T, bool F>
+__device__ __forceinline__ bool pair_term(const Consts &c, const PairSelf &me, const PairCand &cj, bool ok,
+                                          PairTerm &t) {
+    const float4 q = cj.q, pi = me.p;
+    const float pj = cj.p;
+    const float rr = dist2(pi, q);
+    if (!(ok && rr <= c.h2 && rr > c.eps)) return false;
+    if (!(q.w >= 0.0f)) return false;  // neighbour density <= FLT_MIN
+    t.rx = q.x - pi.x;
+    t.ry = q.y - pi.y;
+    t.rz = q.z - pi.z;
+    const float rho_i = me.d.x, p_i = me.d.y, cs_i = me.d.z, iri = me.d.w;
+    const float inv_r = frsq(rr);
+    const float r = rr * inv_r;
+    const float irj = q.w;
+    float hr = fmaxf(c.h - r, 0.0f);
+    t.frag = false;
+    double hrd = 0.0;
+    if constexpr (F) {
+        if (iri > c.fragile_ir || irj > c.fragile_ir) {
+            // Near-isolated pair: h - r in FP64, r from the FP64 r^2 by one
+            // Newton step from the FP32 r (relative error squared: ~1e-14).
+            const double d2 = dist2_d(pi, q), r0 = (double)r;
+            const double rd = __builtin_fma(__builtin_fma(-r0, r0, d2), (double)(0.5f * inv_r), r0);
+            hrd = fmax(c.h_d - rd, 0.0);
+            hr = (float)hrd;
+            t.frag = true;
         }
     }
+    const float cm = c.mCgs * hr * hr * inv_r;  // m gradSpiky(r) / r
+    if (t.frag) {
+        // and its pressure term in FP64: 1/rho^2 of a density near FLT_MIN
+        // overflows FP32 (an infinite force).
+        const double cmd = (double)c.mCgs * hrd * hrd * (double)inv_r;
+        const double midd =
+            __builtin_fma((double)pj, (double)iri * (double)iri, (double)p_i * ((double)irj * (double)irj));
+        t.cprd = cmd * midd;
+    } else {
+        const float mid = __builtin_fmaf(pj, me.iri2, p_i * (irj * irj));
+        t.cpr = cm * mid;
+    }
+    if constexpr (V) {
+        // Approaching pairs only (ux < 0); the others add exact zeros.
+        const float4 vi = me.v, vj = cj.v, dj = cj.d;
+        const float ux =
+            -__builtin_fmaf(vi.z - vj.z, t.rz, __builtin_fmaf(vi.y - vj.y, t.ry, (vi.x - vj.x) * t.rx));
+        const float mu = c.h * ux * frcp(rr + c.visc_eps);
+        const float Pi = -c.nu * (cs_i + dj.z) * mu * frcp(rho_i + dj.x);
+        t.cv = keep(cm * Pi, lanes(ux < 0.0f));
+    }
+    if constexpr (T) {
+        const float4 ni = me.n, nj = cj.n;
+        const float hr3r3 = hr * hr * hr * r * r * r;
+        const float coh = (r > c.halfh) ? hr3r3 : 2.0f * hr3r3 - c.coh_off;
+        const float ch = -c.m2 * coh * inv_r;
+        t.tx = __builtin_fmaf(ch, t.rx, -c.sigma_m * (ni.x - nj.x));
+        t.ty = __builtin_fmaf(ch, t.ry, -c.sigma_m * (ni.y - nj.y));
+        t.tz = __builtin_fmaf(ch, t.rz, -c.sigma_m * (ni.z - nj.z));
+    }
+    return true;
+}
+
+struct PairSums {
+    float Px = 0.f, Py = 0.f, Pz = 0.f;      // pressure sum
+    double Pdx = 0.0, Pdy = 0.0, Pdz = 0.0;  // its near-isolated pairs, in FP64
+    float Qx = 0.f, Qy = 0.f, Qz = 0.f;      // artificial-viscosity part of the viscosity sum
+    float Tx = 0.f, Ty = 0.f, Tz = 0.f;      // cohesion + curvature sum
+    template <bool V, bool T, bool F>
+    __device__ __forceinline__ void add(const PairTerm &t) {
+        if (t.frag) {
+            Pdx = __builtin_fma(t.cprd, (double)t.rx, Pdx);
+            Pdy = __builtin_fma(t.cprd, (double)t.ry, Pdy);
+            Pdz = __builtin_fma(t.cprd, (double)t.rz, Pdz);
+        } else {
+            Px = __builtin_fmaf(t.cpr, t.rx, Px);
+            Py = __builtin_fmaf(t.cpr, t.ry, Py);
+            Pz = __builtin_fmaf(t.cpr, t.rz, Pz);
+        }
+        if constexpr (V) {
+            Qx = __builtin_fmaf(t.cv, t.rx, Qx);
+            Qy = __builtin_fmaf(t.cv, t.ry, Qy);
+            Qz = __builtin_fmaf(t.cv, t.rz, Qz);
+        }
+        if constexpr (T) {
+            Tx += t.tx;
+            Ty += t.ty;
+            Tz += t.tz;
+        }
+    }
+};
+
+// A particle's summed forces; eP: pressure sum of near-isolated pairs (FP64).
+struct Forces {
+    float3 P = {0.f, 0.f, 0.f}, V = {0.f, 0.f, 0.f}, T = {0.f, 0.f, 0.f}, A = {0.f, 0.f, 0.f};
+    double eP[3] = {0.0, 0.0, 0.0};
+};
+
+__device__ __forceinline__ void total_forces(const Consts &c, float4 pi, float4 di, const PairSums &s, Forces &f) {
+    f.P = make_float3(s.Px, s.Py, s.Pz);
+    f.eP[0] = s.Pdx;
+    f.eP[1] = s.Pdy;
+    f.eP[2] = s.Pdz;
+    f.V = make_float3(c.nu * (s.Px + s.Qx), c.nu * (s.Py + s.Qy), c.nu * (s.Pz + s.Qz));
+    // 2 rho0 / (rho_i + rho_i) applied once to the summed tension terms.
+    const float ts = c.sigma * c.rho0 * di.w;
+    f.T = make_float3(ts * s.Tx, ts * s.Ty, ts * s.Tz);
+    if (c.has_adhesion) {
+        // Adhesion toward the walls (fluidphysics.cu:330-350), FP64.
+        const double z = -fmin(box_sdf(c, pi.x, pi.y, pi.z), 0.0) * c.quarter_inv_psize;
+        if (z < 1.0) {
+            double nbv[3];
+            box_normal(c, pi.x, pi.y, pi.z, nbv);
+            const double oz = 1.0 - z;
+            const double k = c.alpha_inv_rho0 * (double)di.x / (oz * oz * oz);
+            f.A = make_float3((float)(k * nbv[0]), (float)(k * nbv[1]), (float)(k * nbv[2]));
+        }
+    }
+}
+
+// Leapfrog integration and boundary clamp of the particle in slot i (src: its
+// state slot), the outputs of the force pass and the far-move flag.
+__device__ __forceinline__ void integrate(const Consts &c, uint32_t i, uint32_t src, float4 pi, float4 vi, float rho,
+                                          const Forces &f, const float4 *__restrict__ A,
+                                          const float4 *__restrict__ Lw, float4 *__restrict__ Pout,
+                                          float4 *__restrict__ Vout, float4 *__restrict__ Aout,
+                                          float4 *__restrict__ Lout, float4 *__restrict__ Fdbg,
+                                          uint32_t *__restrict__ flags, uint32_t move_q) {
     // The viscosity force carries the pressure sum too (nu * (P + Pi)).
+    const float3 fP = f.P, fV = f.V, fT = f.T, fA = f.A;
+    const double *eP = f.eP;
     const double eV[3] = {(double)c.nu * eP[0], (double)c.nu * eP[1], (double)c.nu * eP[2]};
     if (Fdbg) {
         Fdbg[4 * (size_t)i + 0] = make_float4((float)((double)fP.x + eP[0]), (float)((double)fP.y + eP[1]),
@@ -1331,7 +1339,7 @@ __global__ __launch_bounds__(BS) void k_forces(const Consts *__restrict__ cs, co
     const float hx = (float)x, hy = (float)y, hz = (float)z;
     Pout[i] = make_float4(hx, hy, hz, pi.w);
     Lout[i] = make_float4((float)(x - (double)hx), (float)(y - (double)hy), (float)(z - (double)hz), 0.0f);
-    Vout[i] = make_float4((float)vx, (float)vy, (float)vz, di.x);
+    Vout[i] = make_float4((float)vx, (float)vy, (float)vz, rho);
     Aout[i] = make_float4((float)ax, (float)ay, (float)az, 0.0f);
     // Move of the FP32 positions the pair predicates see (the differences
     // are exact in FP64).  Every writer stores the same value; NaN counts
@@ -1339,6 +1347,120 @@ __global__ __launch_bounds__(BS) void k_forces(const Consts *__restrict__ cs, co
     const double move_limit = skin_move_limit(c, skin_frac(move_q));
     const double ex = (double)hx - (double)pi.x, ey = (double)hy - (double)pi.y, ez = (double)hz - (double)pi.z;
     if (!(ex * ex + ey * ey + ez * ez <= move_limit * move_limit)) set_flag(flags, c.scene, kFarMoveByte, 1u);
+}
+
+// The force pass (computeAllForces, fluidphysics.cu:215-352) fused with the
+// leapfrog integrator and boundary clamp (LeapfrogIntegratorOperator,
+// fluidintegrator.cu:11-70).  Out-of-grid particles get zero forces and are
+// still integrated.  Fdbg (may be null) receives the four force components.
+// The pre-XSPH velocity carries the particle's density in w for the XSPH
+// pass, which reads the integrated positions from Pout.  Sets the scene's
+// far-move flag when a particle moved farther than the XSPH skin masks allow.
+template <int BS>
+__global__ __launch_bounds__(BS) void k_forces(const Consts *__restrict__ cs, const uint32_t *__restrict__ chunk,
+                                               uint32_t nslots, const float4 *__restrict__ Ps,
+                                               const float4 *__restrict__ Q, const float *__restrict__ Pr,
+                                               const float4 *__restrict__ Vs, const float4 *__restrict__ A,
+                                               const float4 *__restrict__ Lw, const uint32_t *__restrict__ order,
+                                               const float4 *__restrict__ D,
+                                               const float4 *__restrict__ N, const float *__restrict__ soa,
+                                               const uint32_t *__restrict__ start,
+                                               RowMasks M, int flat, float4 *__restrict__ Pout,
+                                               float4 *__restrict__ Vout, float4 *__restrict__ Aout,
+                                               float4 *__restrict__ Lout,
+                                               float4 *__restrict__ Fdbg, uint32_t *__restrict__ flags,
+                                               const uint32_t *__restrict__ moves, const uint8_t *__restrict__ near) {
+    uint32_t slot0;
+    const Consts *cp = block_scene<BS>(cs, chunk, slot0);
+    if (!cp) return;
+    const Consts &c = *cp;
+    const uint32_t move_q = scene_move_q(moves, c.scene);
+    const uint32_t i = slot0 + threadIdx.x;
+    if (i >= c.first + c.count) return;
+    const uint32_t *st = start + c.cell_base;
+    const uint32_t shift = c.first - st[0];
+    const uint32_t sw = flag_word(flags, c.scene);
+    const uint32_t src = order[i];  // the particle's slot in the state arrays (A, Lw)
+    const float4 pi = Ps[i], vi = Vs[i];
+    const float4 di = D[i];
+    Forces f;
+    if (i < st[c.ncells] + shift) {
+        const PairSelf me{pi, vi, di, c.has_tension ? N[i] : make_float4(0.f, 0.f, 0.f, 0.f), di.w * di.w};
+        PairSums sum;
+        uint32_t b[9], e[9];
+        rows9(c, st, shift, pi, b, e);
+        const RowSource rows{c, st, shift, Ps, soa, moves, nullptr};
+        // One walk per combination of the scene's optional terms, so that a
+        // candidate's loads (V: velocity and density/sound speed; T: normal)
+        // are all issued with its position before any arithmetic.  F: the
+        // scene has near-isolated particles, and a pair with one takes its
+        // h - r in FP64 (a separate walk, so that the other scenes' walks
+        // carry none of its registers' cost).
+        __shared__ uint2 tab[kFlatEntries * BS];
+        auto walk = [&]<bool V, bool T, bool F>() {
+            // (with viscosity the neighbour's pressure comes with its
+            // density record, D.y, instead of a load of its own)
+            using Cand = PairCand;
+            // (two set bits per step in the near-isolated walk: its FP64
+            // terms would otherwise cost every scene's walk registers)
+            walk_rows<BS, F ? 2 : kForceWalkWidth, F ? 0 : kForceLongWidth, 2>(
+                tab, rows, b, e, M, c.use_masks, flat, nslots, i,
+                [&](uint32_t j) { return pair_load<V, T>(Q, Pr, Vs, D, N, j); },
+                [&](const Cand &cj, uint32_t, bool ok) {
+                    PairTerm t;
+                    if (!pair_term<V, T, F>(c, me, cj, ok, t)) return;
+                    sum.template add<V, T, F>(t);
+                });
+        };
+        const bool tension = c.has_tension != 0;
+        auto terms = [&]<bool F>() {
+            if (c.has_visc) {
+                if (tension)
+                    walk.template operator()<true, true, F>();
+                else
+                    walk.template operator()<true, false, F>();
+            } else {
+                if (tension)
+                    walk.template operator()<false, true, F>();
+                else
+                    walk.template operator()<false, false, F>();
+            }
+        };
+        if (flag_set(sw, kFragileByte) && lanes(rows_near(near, b, e)))
+            terms.template operator()<true>();
+        else
+            terms.template operator()<false>();
+        total_forces(c, pi, di, sum, f);
+    }
+    integrate(c, i, src, pi, vi, di.x, f, A, Lw, Pout, Vout, Aout, Lout, Fdbg, flags, move_q);
+}
+
+// A neighbour's integrated position and pre-XSPH velocity (density in w), and
+// its XSPH weight.  A candidate outside h (or with rho_i + rho_j <= FLT_MIN,
+// or passed with ok = false) weighs an exact zero, branch-free.
+struct XsphCand {
+    float4 x, v;
+};
+template <bool F>
+__device__ __forceinline__ float xsph_weight(const Consts &c, float4 xi, float rho_i, const XsphCand &cj, bool ok,
+                                             const float4 *__restrict__ Lw, uint32_t i, uint32_t j) {
+    const float4 q = cj.x;
+    const float rr = dist2(xi, q);
+    const float sr = rho_i + cj.v.w;
+    const uint64_t in = lanes(rr <= c.h2) & lanes(sr > c.eps) & lanes(ok);
+    float t = keep(c.h2 - rr, in);
+    if constexpr (F) {
+        if (sr < c.fragile_sr) {
+            // Near-isolated pair: h^2 - r^2 in FP64 on the double-float
+            // integrated positions (high word in X, low word in Lw).
+            const float4 li = Lw[i], lj = at32(Lw, j);
+            const double dx = ((double)q.x + (double)lj.x) - ((double)xi.x + (double)li.x);
+            const double dy = ((double)q.y + (double)lj.y) - ((double)xi.y + (double)li.y);
+            const double dz = ((double)q.z + (double)lj.z) - ((double)xi.z + (double)li.z);
+            t = keep((float)fmax(c.hh_d - __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx)), 0.0), in);
+        }
+    }
+    return keep(t * t * t * frcp(sr), in);
 }
 
 // 8. XSPH velocity smoothing (correctVelocityXSPH, fluidphysics.cu:355-409):
@@ -1384,39 +1506,18 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(BS >= 512 ? 
     const RowSource rows{c, st, shift, Ps, soa, moves, flag_set(fl, kFarMoveByte) ? Pn : nullptr};
     rows9(c, st, shift, Ps[i], b, e);
     float sx = 0.f, sy = 0.f, sz = 0.f;
-    const float h2 = c.h2, eps = c.eps;
-    // Both loads of a candidate are issued together; a candidate outside h
-    // (or with rho_i + rho_j <= FLT_MIN) adds exact zeros, branch-free.
-    // F: the scene has near-isolated particles (a separate walk, so that the
-    // other scenes' walks carry none of its registers' cost).
-    struct Cand {
-        float4 x, v;
-    };
+    // Both loads of a candidate are issued together.  F: the scene has
+    // near-isolated particles (a separate walk, so that the other scenes'
+    // walks carry none of its registers' cost).
+    using Cand = XsphCand;
     __shared__ uint2 tab[kFlatEntries * BS];
     auto walk = [&]<bool F>() {
         walk_rows<BS, F ? 2 : kXsphWalkWidth, F ? 0 : kXsphWalkWidth, F ? 2 : kXsphRowWidth, !F>(
             tab, rows, b, e, MS, c.use_masks, flat, nslots, i,
             [&](uint32_t j) { return Cand{at32(Pn, j), at32(Vh, j)}; },
             [&](const Cand &cj, uint32_t j, bool ok) {
-                const float4 q = cj.x;
                 const float4 vj = cj.v;
-                const float rr = dist2(xi, q);
-                const float sr = rho_i + vj.w;
-                const uint64_t in = lanes(rr <= h2) & lanes(sr > eps) & lanes(ok);
-                float t = keep(h2 - rr, in);
-                if constexpr (F) {
-                    if (sr < c.fragile_sr) {
-                        // Near-isolated pair: h^2 - r^2 in FP64 on the
-                        // double-float integrated positions (high word in X,
-                        // low word in Lw).
-                        const float4 li = Lw[i], lj = at32(Lw, j);
-                        const double dx = ((double)q.x + (double)lj.x) - ((double)xi.x + (double)li.x);
-                        const double dy = ((double)q.y + (double)lj.y) - ((double)xi.y + (double)li.y);
-                        const double dz = ((double)q.z + (double)lj.z) - ((double)xi.z + (double)li.z);
-                        t = keep((float)fmax(c.hh_d - __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx)), 0.0), in);
-                    }
-                }
-                const float w = keep(t * t * t * frcp(sr), in);
+                const float w = xsph_weight<F>(c, xi, rho_i, cj, ok, Lw, i, j);
                 sx = __builtin_fmaf(w, vj.x - vi.x, sx);
                 sy = __builtin_fmaf(w, vj.y - vi.y, sy);
                 sz = __builtin_fmaf(w, vj.z - vi.z, sz);
@@ -1427,6 +1528,525 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(BS >= 512 ? 
     else
         walk.template operator()<false>();
     Vout[i] = make_float4(vi.x + c.xsph_k * sx, vi.y + c.xsph_k * sy, vi.z + c.xsph_k * sz, 0.0f);
+}
+
+// ---------------------------------------------------------------------------
+// Four lanes per particle.  Below about two waves per SIMD the neighbour
+// passes are bound by each wave's serial chain (row after row, step after
+// step), not by any pipe; there a particle's candidates are spread over four
+// lanes (density / forces / XSPH of the 32,768-particle dam break in its
+// splash: 20.2 / 19.2 / 15.7 us with one lane, 13.5 / 13.0 / 9.8 with four;
+// density / normals / forces / XSPH of the driver's default scene: 28 / 41 /
+// 72 / 90 and 14 / 15 / 25 / 30).  Sums stay in slot order, so every bit is that of the one-lane
+// kernels: each lane computes the terms of its candidates, then the quad's
+// lanes take turns adding theirs to the running sums, the result of each turn
+// broadcast to the quad (DPP).
+constexpr int kQuadBlock = 256;                 // 64 particles per workgroup
+constexpr uint32_t kQuadParts = kQuadBlock / 4;
+constexpr uint32_t kQuadList = 128;             // neighbour slots of a particle listed at a time
+constexpr uint32_t kQuadStride = kQuadList + 4;  // (lists of a wave's particles start in different banks)
+
+template <int R>
+__device__ __forceinline__ uint32_t quad_get(uint32_t v) {  // lane R's value
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, R * 0x55, 0xF, 0xF, true);
+}
+template <int R>
+__device__ __forceinline__ float quad_get(float v) {
+    return __uint_as_float(quad_get<R>(__float_as_uint(v)));
+}
+template <int R>
+__device__ __forceinline__ double quad_get(double v) {
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    return __longlong_as_double((long long)((uint64_t)quad_get<R>((uint32_t)(u >> 32)) << 32 |
+                                            quad_get<R>((uint32_t)u)));
+}
+__device__ __forceinline__ uint32_t quad_or(uint32_t v) {
+    v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);  // lanes 1 0 3 2
+    v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true);  // lanes 2 3 0 1
+    return v;
+}
+// Orders a wave's LDS accesses of different lanes (a quad is inside one wave).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// First slots and lengths of the rows q, q + 4 and (lane 0) 8 of lane q.
+struct QuadRows {
+    uint32_t s[3], len[3];
+};
+__device__ __forceinline__ QuadRows quad_rows(const Consts &c, const uint32_t *__restrict__ start, uint32_t shift,
+                                              float4 pc, uint32_t q) {
+    QuadRows w;
+#pragma unroll
+    for (uint32_t k = 0; k < 3u; ++k) {
+        const uint32_t r = q + 4u * k;
+        const uint2 x = row_span(c, start, shift, pc, r < 9u ? r : 4u);
+        w.s[k] = x.x;
+        w.len[k] = r < 9u ? x.y - x.x : 0u;
+    }
+    return w;
+}
+__device__ __forceinline__ bool quad_near(const uint8_t *__restrict__ near, const QuadRows &w) {
+    uint32_t any = 0u;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        if (w.len[k])
+            for (uint32_t a = w.s[k] / kNearBlock; a <= (w.s[k] + w.len[k] - 1u) / kNearBlock; ++a) any |= near[a];
+    return any != 0u;
+}
+
+// Eight candidates [s, s + 8) of a lane (n of them in its row): those within
+// the skin radius (slots' planes, as skin_word) or, with src.moved, within h
+// of the integrated position pc (as moved_word); every one when !use.
+__device__ __forceinline__ uint32_t skin_byte(const RowSource &src, uint32_t nslots, bool use, float4 pc, float h2s,
+                                              uint32_t s, uint32_t n, uint32_t i) {
+    uint32_t m = 0xFFu;
+    if (use && src.moved) {
+        float4 x[8];
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; ++k) x[k] = at32(src.moved, k < n ? s + k : i);
+        m = 0u;
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; ++k) m |= dist2(pc, x[k]) <= src.c.h2 ? 1u << k : 0u;
+    } else if (use) {
+        const __amdgpu_buffer_rsrc_t px = plane_buffer(src.soa, nslots), py = plane_buffer(src.soa + nslots, nslots),
+                                     pz = plane_buffer(src.soa + 2 * (size_t)nslots, nslots);
+        const uint32_t vo = s * (uint32_t)sizeof(float);
+        const float4 X[2] = {load4(px, vo, 0u), load4(px, vo, 16u)}, Y[2] = {load4(py, vo, 0u), load4(py, vo, 16u)},
+                     Z[2] = {load4(pz, vo, 0u), load4(pz, vo, 16u)};
+        m = 0u;
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; ++k) {
+            const float dx = (&X[k / 4].x)[k % 4] - pc.x, dy = (&Y[k / 4].x)[k % 4] - pc.y,
+                        dz = (&Z[k / 4].x)[k % 4] - pc.z;
+            const float rs = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, -h2s)));
+            m |= (__float_as_uint(rs) >> 31) << k;
+        }
+    }
+    if (n < 8u) m &= (1u << n) - 1u;
+    if (i - s < 8u) m &= ~(1u << (i - s));  // the particle itself is no candidate
+    return m;
+}
+
+// Lists the particle's candidates in slot order and walks the list sixteen at
+// a time: lane q takes entries 4q .. 4q + 3.  Where the stored mask words are
+// all a wave's particles have (rows of at most 96 slots), each lane lists the
+// set bits of its own rows, in parts of kQuadList entries; else the quad goes
+// through the rows together, eight slots of every mask word per lane (words
+// not stored are tested, every slot taken when !use), and walks when another
+// word may not fit.  term(candidate, slot, ok) gives a candidate's term (zero
+// when !ok or it adds nothing), sums.add(term) adds it, sums.get<R>() is lane
+// R's.
+template <class Sums, class Ld, class Fn>
+__device__ __forceinline__ void walk_quad(uint32_t *__restrict__ list, const RowSource &src, const QuadRows &w,
+                                          const RowMasks &mask, bool use, uint32_t nslots, uint32_t i, uint32_t q,
+                                          Sums &sums, Ld &&ld, Fn &&term) {
+    uint64_t w01[3];
+    uint32_t w2[3], at[3], total = 0u;
+    bool tested = false;  // some word is not stored
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const uint32_t r = q + 4u * (uint32_t)k;
+        const size_t m = (size_t)(r < 9u ? r : 4u) * nslots + i;
+        w01[k] = w.len[k] ? row_mask64(mask, m, w.len[k]) : 0ull;
+        w2[k] = w.len[k] > 64u ? mask.w32[m] : 0u;
+        tested = tested || w.len[k] > 96u;
+    }
+    const bool words = __ballot(tested || src.moved || !use) == 0ull;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {  // each row's place in the list: rows 0..3 (one per lane), then 4..7, then 8
+        const uint32_t cnt = (uint32_t)__popcll(w01[k]) + (uint32_t)__popc(w2[k]);
+        const uint32_t c0 = quad_get<0>(cnt), c1 = quad_get<1>(cnt), c2 = quad_get<2>(cnt), c3 = quad_get<3>(cnt);
+        at[k] = total + (q > 0u ? c0 : 0u) + (q > 1u ? c1 : 0u) + (q > 2u ? c2 : 0u);
+        total += c0 + c1 + c2 + c3;
+    }
+    const auto put = [&](uint32_t &idx, uint32_t s, uint32_t m) {
+        while (m) {
+            if (idx < kQuadList) list[idx] = s + (uint32_t)__builtin_ctz(m);
+            m &= m - 1u;
+            ++idx;
+        }
+    };
+    uint32_t base = 0u;             // words: entries walked so far
+    uint32_t row = 0u, word = 0u;   // else the next word (wave-uniform)
+    bool more = true;
+#pragma unroll 1
+    while (more) {
+        uint32_t n = 0u;  // entries listed
+        wave_lds_sync();  // the last part's entries have been read
+        if (words) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                uint32_t idx = at[k] - base;  // (entries of earlier parts wrap round past kQuadList)
+                put(idx, w.s[k], (uint32_t)w01[k]);
+                put(idx, w.s[k] + 32u, (uint32_t)(w01[k] >> 32));
+                put(idx, w.s[k] + 64u, w2[k]);
+            }
+            n = base < total ? total - base : 0u;
+            n = n < kQuadList ? n : kQuadList;
+            base += kQuadList;
+            more = __ballot(base < total) != 0ull;
+        } else {
+            const float4 pc = at32(src.pos, i);
+            const float4 xt = src.moved ? at32(src.moved, i) : pc;
+            const float h2s = skin_h2s(src.c, skin_frac(scene_move_q(src.moves, src.c.scene)));
+            uint2 cur = row_span(src.c, src.st, src.shift, pc, row);
+            bool full = false;
+#pragma unroll 1
+            while (row < 9u && !full) {
+                const uint2 nxt = row_span(src.c, src.st, src.shift, pc, row < 8u ? row + 1u : 8u);
+                const uint32_t len = cur.y - cur.x;
+#pragma unroll 1
+                for (; __ballot(32u * word < len); ++word) {
+                    full = __ballot(n + 32u > kQuadList) != 0ull;
+                    if (full) break;
+                    const uint32_t o = 32u * word + 8u * q;
+                    uint32_t m = 0u;
+                    if (o < len) {
+                        if (use && !src.moved && word < 3u) {
+                            const size_t t = (size_t)row * nslots + i;
+                            m = (word < 2u ? (uint32_t)(row_mask64(mask, t, len) >> (32u * word)) : mask.w32[t]) >>
+                                    (8u * q) & 0xFFu;
+                        } else {
+                            m = skin_byte(src, nslots, use, xt, h2s, cur.x + o, len - o, i);
+                        }
+                    }
+                    const uint32_t cnt = (uint32_t)__popc(m);
+                    const uint32_t c0 = quad_get<0>(cnt), c1 = quad_get<1>(cnt), c2 = quad_get<2>(cnt),
+                                   c3 = quad_get<3>(cnt);
+                    uint32_t idx = n + (q > 0u ? c0 : 0u) + (q > 1u ? c1 : 0u) + (q > 2u ? c2 : 0u);
+                    put(idx, cur.x + o, m);
+                    n += c0 + c1 + c2 + c3;
+                }
+                if (!full) {
+                    word = 0u;
+                    ++row;
+                    cur = nxt;
+                }
+            }
+            more = row < 9u;
+        }
+        wave_lds_sync();
+#pragma unroll 1
+        for (uint32_t k0 = 0u; k0 < n; k0 += 16u) {
+            const uint32_t mine = k0 + 4u * q;
+            const uint4 e = *reinterpret_cast<const uint4 *>(list + mine);
+            const uint32_t es[4] = {e.x, e.y, e.z, e.w};
+            uint32_t j[4];
+            bool ok[4];
+            decltype(ld(0u)) a[4];
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; ++k) {
+                ok[k] = mine + k < n;
+                j[k] = ok[k] ? es[k] : i;
+                a[k] = ld(j[k]);
+            }
+            decltype(term(a[0], 0u, true)) t[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) t[k] = term(a[k], j[k], ok[k]);
+            const auto turn = [&]<int R>() {
+                Sums mine4 = sums;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) mine4.add(t[k]);
+                sums = mine4.template get<R>();
+            };
+            turn.template operator()<0>();
+            turn.template operator()<1>();
+            turn.template operator()<2>();
+            turn.template operator()<3>();
+        }
+    }
+}
+
+// Scene, slot and lane of a four-lane kernel's thread; false: nothing to do.
+__device__ __forceinline__ const Consts *quad_scene(const Consts *__restrict__ cs, const uint32_t *__restrict__ chunk,
+                                                    uint32_t &i, uint32_t &q) {
+    uint32_t slot0;
+    const Consts *cp = block_scene<kQuadParts>(cs, chunk, slot0);
+    i = slot0 + (threadIdx.x >> 2);
+    q = threadIdx.x & 3u;
+    return cp;
+}
+
+// k_density for few particles.  The quad scans a row sixteen slots at a time,
+// four per lane, and the next row's first 32 slots are loaded before a row is
+// tested.
+__global__ __launch_bounds__(kQuadBlock) void k_density_quad(
+    const Consts *__restrict__ cs, const uint32_t *__restrict__ chunk, uint32_t nslots, const float4 *__restrict__ Ps,
+    const float *__restrict__ soa, const uint32_t *__restrict__ start, float4 *__restrict__ D, float4 *__restrict__ Q,
+    float *__restrict__ Pr, RowMasks MS, uint32_t *__restrict__ flags, const uint32_t *__restrict__ moves,
+    uint8_t *__restrict__ near) {
+    uint32_t i, q;
+    const Consts *cp = quad_scene(cs, chunk, i, q);
+    if (!cp) return;
+    const Consts &c = *cp;
+    const float h2s = skin_h2s(c, skin_frac(scene_move_q(moves, c.scene)));
+    if (i == c.first && q == 0u) set_flag(flags, c.scene, kFarMoveByte, 0u);
+    if (i >= c.first + c.count) return;
+    const uint32_t *st = start + c.cell_base;
+    const uint32_t shift = c.first - st[0];
+    if (i >= st[c.ncells] + shift) {
+        if (q == 0u) D[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        return;
+    }
+    const float4 pi = Ps[i];
+    uint32_t b[9], e[9];
+    rows9(c, st, shift, pi, b, e);
+    const float nh2s = -h2s, ninv_h2 = -c.inv_h2;
+    const float c1 = (c.h2 - h2s) * c.inv_h2;
+    const __amdgpu_buffer_rsrc_t px = plane_buffer(soa, nslots), py = plane_buffer(soa + nslots, nslots),
+                                 pz = plane_buffer(soa + 2 * (size_t)nslots, nslots);
+    struct Group {
+        float4 X, Y, Z;
+    };
+    const auto load = [&](uint32_t s) {  // slots [s, s + 4) of the planes
+        const uint32_t vo = s * (uint32_t)sizeof(float);
+        return Group{load4(px, vo, 0u), load4(py, vo, 0u), load4(pz, vo, 0u)};
+    };
+    float S = 0.0f;
+    // Slots [k0, k0 + 4) of row r, this lane's; returns the sixteen mask bits
+    // of the quad's slots.
+    const auto scan = [&](const Group &g, int r, uint32_t c0, uint32_t len, uint32_t kself) -> uint32_t {
+        const float X[4] = {g.X.x, g.X.y, g.X.z, g.X.w}, Y[4] = {g.Y.x, g.Y.y, g.Y.z, g.Y.w},
+                    Z[4] = {g.Z.x, g.Z.y, g.Z.z, g.Z.w};
+        const uint32_t k0 = c0 + 4u * q;
+        uint32_t bits = 0u;
+        float t[4], tt[4];
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k) {
+            const float dx = X[k] - pi.x, dy = Y[k] - pi.y, dz = Z[k] - pi.z;
+            float rs = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, nh2s)));
+            if (r == 4) rs = (k0 + k == kself) ? 1.0f : rs;
+            rs = (k0 + k < len) ? rs : 1.0f;
+            t[k] = fminf(fmaxf(__builtin_fmaf(rs, ninv_h2, c1), 0.0f), 1.0f);
+            tt[k] = t[k] * t[k];
+            bits |= (__float_as_uint(rs) >> 31) << k;
+        }
+        const auto turn = [&]<int R>() {
+            float mine = S;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) mine = __builtin_fmaf(tt[k], t[k], mine);
+            S = quad_get<R>(mine);
+        };
+        turn.template operator()<0>();
+        turn.template operator()<1>();
+        turn.template operator()<2>();
+        turn.template operator()<3>();
+        return quad_or(bits << (4u * q));
+    };
+    Group g0 = load(b[0] + 4u * q), g1 = load(b[0] + 16u + 4u * q);
+#pragma unroll
+    for (int r = 0; r < 9; ++r) {
+        const uint32_t len = e[r] - b[r], kself = i - b[r];
+        const Group a0 = g0, a1 = g1;
+        if (r < 8) {
+            g0 = load(b[r + 1] + 4u * q);
+            g1 = load(b[r + 1] + 16u + 4u * q);
+        }
+        uint32_t s0 = 0u, s1 = 0u, s2 = 0u;
+        if (len > 0u) s0 = scan(a0, r, 0u, len, kself);
+        if (len > 16u) s0 |= scan(a1, r, 16u, len, kself) << 16;
+#pragma unroll 1
+        for (uint32_t c0 = 32u; c0 < len; c0 += 16u) {
+            const uint32_t m = scan(load(b[r] + c0 + 4u * q), r, c0, len, kself) << (c0 & 16u);
+            if (c0 < 64u)
+                s1 |= m;
+            else if (c0 < 96u)
+                s2 |= m;
+        }
+        if (q == 0u) {
+            const size_t at = (size_t)r * nslots + i;
+            if (len <= 32u)
+                MS.w32[at] = s0;
+            else
+                MS.w64[at] = (uint64_t)s1 << 32 | s0;
+            if (len > 64u) MS.w32[at] = s2;
+        }
+    }
+    if (q != 0u) return;
+    S = S < c.fragile_S ? (float)(near_isolated_sum(c, b, e, Ps, MS, nslots, i, pi) * c.mC6_d) : S * c.mC6h6;
+    density_finish(c, i, pi, S, D, Q, Pr, flags, near);
+}
+
+struct Vec3Sum {
+    float x = 0.f, y = 0.f, z = 0.f;
+    __device__ __forceinline__ void add(float4 t) {  // t.w (t.x, t.y, t.z)
+        x = __builtin_fmaf(t.w, t.x, x);
+        y = __builtin_fmaf(t.w, t.y, y);
+        z = __builtin_fmaf(t.w, t.z, z);
+    }
+    template <int R>
+    __device__ __forceinline__ Vec3Sum get() const {
+        Vec3Sum s;
+        s.x = quad_get<R>(x);
+        s.y = quad_get<R>(y);
+        s.z = quad_get<R>(z);
+        return s;
+    }
+};
+
+__global__ __launch_bounds__(kQuadBlock) void k_normals_quad(
+    const Consts *__restrict__ cs, const uint32_t *__restrict__ chunk, uint32_t nslots, const float4 *__restrict__ Q,
+    const float *__restrict__ soa, const uint32_t *__restrict__ start, RowMasks M, int all,
+    const uint32_t *__restrict__ flags, const uint32_t *__restrict__ moves, const uint8_t *__restrict__ near,
+    float4 *__restrict__ N) {
+    __shared__ __align__(16) uint32_t lists[kQuadParts * kQuadStride];
+    uint32_t i, q;
+    const Consts *cp = quad_scene(cs, chunk, i, q);
+    if (!cp || (cp->lazy_normal && !all)) return;
+    const Consts &c = *cp;
+    if (i >= c.first + c.count) return;
+    const uint32_t *st = start + c.cell_base;
+    const uint32_t shift = c.first - st[0];
+    if (i >= st[c.ncells] + shift) {
+        if (q == 0u) N[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        return;
+    }
+    const float4 pi = Q[i];
+    const QuadRows rows = quad_rows(c, st, shift, pi, q);
+    const RowSource src{c, st, shift, Q, soa, moves, nullptr};
+    Vec3Sum sum;
+    auto walk = [&]<bool F>() {
+        walk_quad(
+            lists + (threadIdx.x >> 2) * kQuadStride, src, rows, M, c.use_masks != 0, nslots, i, q, sum,
+            [&](uint32_t j) { return at32(Q, j); },
+            [&](const float4 &cand, uint32_t, bool ok) {
+                const float w = normal_weight<F>(c, pi, cand, dist2(pi, cand), ok);
+                return make_float4(pi.x - cand.x, pi.y - cand.y, pi.z - cand.z, w);
+            });
+    };
+    if (flag_set(flag_word(flags, c.scene), kFragileByte) && lanes(quad_near(near, rows)))
+        walk.template operator()<true>();
+    else
+        walk.template operator()<false>();
+    if (q == 0u) N[i] = make_float4(c.hmCg6 * sum.x, c.hmCg6 * sum.y, c.hmCg6 * sum.z, 0.0f);
+}
+
+template <bool V, bool T, bool F>
+struct QuadPairSums : PairSums {
+    __device__ __forceinline__ void add(const PairTerm &t) { PairSums::template add<V, T, F>(t); }
+    template <int R>
+    __device__ __forceinline__ QuadPairSums get() const {
+        QuadPairSums s;
+        s.Px = quad_get<R>(Px);
+        s.Py = quad_get<R>(Py);
+        s.Pz = quad_get<R>(Pz);
+        if constexpr (F) {
+            s.Pdx = quad_get<R>(Pdx);
+            s.Pdy = quad_get<R>(Pdy);
+            s.Pdz = quad_get<R>(Pdz);
+        }
+        if constexpr (V) {
+            s.Qx = quad_get<R>(Qx);
+            s.Qy = quad_get<R>(Qy);
+            s.Qz = quad_get<R>(Qz);
+        }
+        if constexpr (T) {
+            s.Tx = quad_get<R>(Tx);
+            s.Ty = quad_get<R>(Ty);
+            s.Tz = quad_get<R>(Tz);
+        }
+        return s;
+    }
+};
+
+__global__ __launch_bounds__(kQuadBlock) void k_forces_quad(
+    const Consts *__restrict__ cs, const uint32_t *__restrict__ chunk, uint32_t nslots, const float4 *__restrict__ Ps,
+    const float4 *__restrict__ Q, const float *__restrict__ Pr, const float4 *__restrict__ Vs,
+    const float4 *__restrict__ A, const float4 *__restrict__ Lw, const uint32_t *__restrict__ order,
+    const float4 *__restrict__ D, const float4 *__restrict__ N, const float *__restrict__ soa,
+    const uint32_t *__restrict__ start, RowMasks M, float4 *__restrict__ Pout, float4 *__restrict__ Vout,
+    float4 *__restrict__ Aout, float4 *__restrict__ Lout, float4 *__restrict__ Fdbg, uint32_t *__restrict__ flags,
+    const uint32_t *__restrict__ moves, const uint8_t *__restrict__ near) {
+    __shared__ __align__(16) uint32_t lists[kQuadParts * kQuadStride];
+    uint32_t i, q;
+    const Consts *cp = quad_scene(cs, chunk, i, q);
+    if (!cp) return;
+    const Consts &c = *cp;
+    const uint32_t move_q = scene_move_q(moves, c.scene);
+    if (i >= c.first + c.count) return;
+    const uint32_t *st = start + c.cell_base;
+    const uint32_t shift = c.first - st[0];
+    const float4 pi = Ps[i], vi = Vs[i], di = D[i];
+    Forces f;
+    if (i < st[c.ncells] + shift) {
+        const PairSelf me{pi, vi, di, c.has_tension ? N[i] : make_float4(0.f, 0.f, 0.f, 0.f), di.w * di.w};
+        const QuadRows rows = quad_rows(c, st, shift, pi, q);
+        const RowSource src{c, st, shift, Ps, soa, moves, nullptr};
+        PairSums sum;
+        auto walk = [&]<bool V, bool T, bool F>() {
+            QuadPairSums<V, T, F> s;
+            walk_quad(
+                lists + (threadIdx.x >> 2) * kQuadStride, src, rows, M, c.use_masks != 0, nslots, i, q, s,
+                [&](uint32_t j) { return pair_load<V, T>(Q, Pr, Vs, D, N, j); },
+                [&](const PairCand &cj, uint32_t, bool ok) {
+                    PairTerm t = {};
+                    if (!pair_term<V, T, F>(c, me, cj, ok, t)) t = PairTerm{};
+                    return t;
+                });
+            sum = s;
+        };
+        auto terms = [&]<bool F>() {
+            if (c.has_visc) {
+                if (c.has_tension)
+                    walk.template operator()<true, true, F>();
+                else
+                    walk.template operator()<true, false, F>();
+            } else {
+                if (c.has_tension)
+                    walk.template operator()<false, true, F>();
+                else
+                    walk.template operator()<false, false, F>();
+            }
+        };
+        if (flag_set(flag_word(flags, c.scene), kFragileByte) && lanes(quad_near(near, rows)))
+            terms.template operator()<true>();
+        else
+            terms.template operator()<false>();
+        total_forces(c, pi, di, sum, f);
+    }
+    if (q == 0u) integrate(c, i, order[i], pi, vi, di.x, f, A, Lw, Pout, Vout, Aout, Lout, Fdbg, flags, move_q);
+}
+
+__global__ __launch_bounds__(kQuadBlock) void k_xsph_quad(
+    const Consts *__restrict__ cs, const uint32_t *__restrict__ chunk, uint32_t nslots, const float4 *__restrict__ Ps,
+    const float4 *__restrict__ Pn, const float4 *__restrict__ Vh, const float4 *__restrict__ Lw,
+    const float *__restrict__ soa, const uint32_t *__restrict__ start, RowMasks MS, const uint32_t *__restrict__ flags,
+    const uint32_t *__restrict__ moves, const uint8_t *__restrict__ near, float4 *__restrict__ Vout) {
+    __shared__ __align__(16) uint32_t lists[kQuadParts * kQuadStride];
+    uint32_t i, q;
+    const Consts *cp = quad_scene(cs, chunk, i, q);
+    if (!cp) return;
+    const Consts &c = *cp;
+    if (i >= c.first + c.count) return;
+    const uint32_t *st = start + c.cell_base;
+    const uint32_t shift = c.first - st[0];
+    const float4 vi = Vh[i];
+    if (i >= st[c.ncells] + shift) {
+        if (q == 0u) Vout[i] = make_float4(vi.x, vi.y, vi.z, 0.0f);
+        return;
+    }
+    const uint32_t fl = flag_word(flags, c.scene);
+    const float4 xi = Pn[i];
+    const QuadRows rows = quad_rows(c, st, shift, Ps[i], q);
+    const RowSource src{c, st, shift, Ps, soa, moves, flag_set(fl, kFarMoveByte) ? Pn : nullptr};
+    Vec3Sum sum;
+    auto walk = [&]<bool F>() {
+        walk_quad(
+            lists + (threadIdx.x >> 2) * kQuadStride, src, rows, MS, c.use_masks != 0, nslots, i, q, sum,
+            [&](uint32_t j) { return XsphCand{at32(Pn, j), at32(Vh, j)}; },
+            [&](const XsphCand &cj, uint32_t j, bool ok) {
+                const float w = xsph_weight<F>(c, xi, vi.w, cj, ok, Lw, i, j);
+                return make_float4(cj.v.x - vi.x, cj.v.y - vi.y, cj.v.z - vi.z, w);
+            });
+    };
+    if (flag_set(fl, kFragileByte) && lanes(quad_near(near, rows)))
+        walk.template operator()<true>();
+    else
+        walk.template operator()<false>();
+    if (q == 0u)
+        Vout[i] = make_float4(vi.x + c.xsph_k * sum.x, vi.y + c.xsph_k * sum.y, vi.z + c.xsph_k * sum.z, 0.0f);
 }
 
 // ---------------------------------------------------------------------------
@@ -1679,6 +2299,16 @@ static inline void with_bs(int bs, F &&body) {
     }
 }
 
+// Whether the neighbour passes take four lanes per particle: launches of so
+// few slots that one lane each leaves the chip's 1,024 SIMDs with less than a
+// wave or two.  Measured, a substep with one / four lanes: plain fluid, 32,768
+// particles 58 / 48 us at rest and 80 / 60 in the splash, 65,000 68 / 71 and
+// 91 / 91, 98,000 72 / 84 and 96 / 110; with viscosity or tension, whose
+// pairs cost twice as much, 10,000 particles 190 / 90, 65,000 174 / 140 and
+// 308 / 224, 98,000 162 / 157 and 365 / 355, 131,000 521 / 519.
+constexpr uint32_t kQuadSlots = 49152, kQuadSlotsFull = 98304;
+static inline bool use_quads(const PoolView &pv) { return pv.nlaunch <= (pv.full ? kQuadSlotsFull : kQuadSlots); }
+
 bool valid_block_size(int bs) { return bs == 128 || bs == 256 || bs == 512; }
 
 void launch_hash(const Launch &L, const PoolView &pv, const float4 *P, uint32_t *keys, uint32_t *ranks,
@@ -1716,6 +2346,11 @@ void launch_gather(const Launch &L, const PoolView &pv, const uint32_t *slot_src
 void launch_density(const Launch &L, const PoolView &pv, int bs, const float4 *Ps, const float *soa,
                     const uint32_t *start, float4 *D, float4 *Q, float *Pr, RowMasks MS, uint32_t *flags,
                     const uint32_t *moves) {
+    if (use_quads(pv)) {
+        LF_GO(L, k_density_quad, pv.nlaunch / kQuadParts, kQuadBlock, L.a, L.b, pv.cs, pv.chunk, pv.nslots, Ps, soa,
+              start, D, Q, Pr, MS, flags, moves, pv.near);
+        return;
+    }
     with_bs(bs, [&]<int BS>() {
         LF_GO(L, k_density<BS>, pv.nlaunch / BS, BS, L.a, L.b, pv.cs, pv.chunk, pv.nslots, Ps, soa, start, D, Q, Pr,
               MS, flags, moves, pv.near);
@@ -1725,6 +2360,11 @@ void launch_density(const Launch &L, const PoolView &pv, int bs, const float4 *P
 void launch_normals(const Launch &L, const PoolView &pv, int bs, int flat, bool all, const float4 *Q,
                     const float *soa, const uint32_t *start, RowMasks M, const uint32_t *flags, const uint32_t *moves,
                     float4 *N) {
+    if (use_quads(pv)) {
+        LF_GO(L, k_normals_quad, pv.nlaunch / kQuadParts, kQuadBlock, L.a, L.b, pv.cs, pv.chunk, pv.nslots, Q, soa,
+              start, M, all ? 1 : 0, flags, moves, pv.near, N);
+        return;
+    }
     with_bs(bs, [&]<int BS>() {
         LF_GO(L, k_normals<BS>, pv.nlaunch / BS, BS, L.a, L.b, pv.cs, pv.chunk, pv.nslots, Q, soa, start, M,
               flat, all ? 1 : 0, flags, moves, pv.near, N);
@@ -1736,6 +2376,11 @@ void launch_forces(const Launch &L, const PoolView &pv, int bs, int flat, const 
                    const float4 *D, const float4 *N, const float *soa, const uint32_t *start, RowMasks M,
                    float4 *Pout, float4 *Vout, float4 *Aout, float4 *Lout, float4 *Fdbg, uint32_t *flags,
                    const uint32_t *moves) {
+    if (use_quads(pv)) {
+        LF_GO(L, k_forces_quad, pv.nlaunch / kQuadParts, kQuadBlock, L.a, L.b, pv.cs, pv.chunk, pv.nslots, Ps, Q, Pr,
+              Vs, A, Lw, order, D, N, soa, start, M, Pout, Vout, Aout, Lout, Fdbg, flags, moves, pv.near);
+        return;
+    }
     with_bs(bs, [&]<int BS>() {
         LF_GO(L, k_forces<BS>, pv.nlaunch / BS, BS, L.a, L.b, pv.cs, pv.chunk, pv.nslots, Ps, Q, Pr, Vs, A, Lw, order,
               D, N, soa, start, M, flat, Pout, Vout, Aout, Lout, Fdbg, flags, moves, pv.near);
@@ -1745,6 +2390,11 @@ void launch_forces(const Launch &L, const PoolView &pv, int bs, int flat, const 
 void launch_xsph(const Launch &L, const PoolView &pv, int bs, int flat, const float4 *Ps, const float4 *Pn,
                  const float4 *Vh, const float4 *Lw, const float *soa, const uint32_t *start, RowMasks MS,
                  const uint32_t *flags, const uint32_t *moves, float4 *Vout) {
+    if (use_quads(pv)) {
+        LF_GO(L, k_xsph_quad, pv.nlaunch / kQuadParts, kQuadBlock, L.a, L.b, pv.cs, pv.chunk, pv.nslots, Ps, Pn, Vh,
+              Lw, soa, start, MS, flags, moves, pv.near, Vout);
+        return;
+    }
     with_bs(bs, [&]<int BS>() {
         LF_GO(L, k_xsph<BS>, pv.nlaunch / BS, BS, L.a, L.b, pv.cs, pv.chunk, pv.nslots, Ps, Pn, Vh, Lw, soa,
               start, MS, flat, flags, moves, pv.near, Vout);

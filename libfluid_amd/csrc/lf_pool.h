@@ -144,7 +144,8 @@ class Pool {
     template <class Fn>
     void timed(int kind, Fn &&launch);
     void drop_graph();
-    PoolView view() const { return PoolView{d_cs_, d_chunk_, nslots_, span_slots_, near_}; }
+    bool any_full() const;
+    PoolView view() const { return PoolView{d_cs_, d_chunk_, nslots_, span_slots_, near_, any_full()}; }
     void set_spans();
 
     int device_ = 0;
@@ -196,6 +197,7 @@ class Pool {
     hipGraphExec_t graph_exec_[2] = {};
     int parity_ = 0;              // which pairing is current (toggled by advance_state)
     bool graph_normals_ = false;  // the captured substeps have the normals pass
+    bool graph_full_ = false;     // and a scene with viscosity or tension
     std::vector<std::pair<uint32_t, uint32_t>> graph_paused_;  // and carry these paused scenes' slots
     std::pair<uint32_t, uint32_t> graph_span_{0, 0};         // and cover these spans
 

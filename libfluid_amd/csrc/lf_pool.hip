@@ -532,6 +532,12 @@ bool Pool::any_separate_normals() const {
     return false;
 }
 
+bool Pool::any_full() const {
+    for (const SceneRec &s : scenes_)
+        if (s.live && s.active && (s.params.viscosity != 0.0f || s.params.surface_tension != 0.0f)) return true;
+    return false;
+}
+
 // Hash, scan, provisional scatter and stable gather of the state positions
 // and velocities (P0, V0) into cell order (P1, V1); ranks_ then holds, per
 // cell-order slot, the particle's state slot (the force pass reads A0 and L0
@@ -620,7 +626,7 @@ int Pool::run_substeps(uint32_t substeps) {
     }
     const std::pair<uint32_t, uint32_t> span{span_slots_, span_buckets_};
     if ((graph_exec_[0] || graph_exec_[1]) &&
-        (graph_normals_ != any_separate_normals() || graph_paused_ != paused_ranges() || graph_span_ != span))
+        (graph_normals_ != any_separate_normals() || graph_full_ != any_full() || graph_paused_ != paused_ranges() || graph_span_ != span))
         drop_graph();
     for (uint32_t k = 0; k < substeps; ++k) {
         hipGraphExec_t &ge = graph_exec_[parity_];
@@ -641,6 +647,7 @@ int Pool::run_substeps(uint32_t substeps) {
             }
             graph_[parity_] = g;
             graph_normals_ = any_separate_normals();
+            graph_full_ = any_full();
             graph_paused_ = paused_ranges();
             graph_span_ = span;
         }
