@@ -14,7 +14,7 @@ constexpr uint32_t kMaxParticles = 1u << 28;  // pool slots: 16-byte records add
 // Stable placement by (cell, id): a bucket of at most kRankDirectMax
 // particles is ranked by id directly (each member counts the smaller ids,
 // O(size^2) per bucket); a larger one is sorted by id as a segment (LSD
-// radix sort, O(size) per pass, in k_gather).
+// radix sort, O(size) per pass, k_sort_segments).
 constexpr uint32_t kRankDirectMax = 512;
 constexpr int kScanPerThread = 4;             // cell-count scan: entries per thread (one 16-byte load)
 constexpr int kScanTile = kBlock * kScanPerThread;
@@ -389,9 +389,8 @@ __device__ __forceinline__ float frsq(float x) { return __builtin_amdgcn_rsqf(x)
 // Workgroup index remapped so that each XCD (which takes workgroups
 // round-robin) processes one contiguous range of particles: neighbours of a
 // particle then mostly live in the same XCD's L2.
-// (The launch's first `skip` workgroups, a multiple of 8, have other work.)
-__device__ __forceinline__ uint32_t xcd_block(uint32_t skip) {
-    const uint32_t nb = gridDim.x - skip, b = blockIdx.x - skip;
+__device__ __forceinline__ uint32_t xcd_block() {
+    const uint32_t nb = gridDim.x, b = blockIdx.x;
     const uint32_t q = nb >> 3, r = nb & 7u, x = b & 7u, k = b >> 3;
     return x * q + (x < r ? x : r) + k;
 }
@@ -402,10 +401,9 @@ __device__ __forceinline__ uint32_t xcd_block(uint32_t skip) {
 // workgroup never straddles two scenes and the lookup is uniform.
 template <int BS>
 __device__ __forceinline__ const Consts *block_scene(const Consts *__restrict__ cs,
-                                                     const uint32_t *__restrict__ chunk, uint32_t &slot0,
-                                                     uint32_t skip = 0u) {
+                                                     const uint32_t *__restrict__ chunk, uint32_t &slot0) {
     static_assert(kChunk % BS == 0, "block size must divide the chunk");
-    slot0 = xcd_block(skip) * (uint32_t)BS;
+    slot0 = xcd_block() * (uint32_t)BS;
     const uint32_t s = chunk[slot0 / kChunk];
     return s == kNoScene ? nullptr : cs + s;
 }

@@ -41,18 +41,18 @@ void launch_hash(const Launch &L, const PoolView &pv, const float4 *P, uint32_t 
 // Exclusive scan of counts[0, m) into start[0, m] (start[m] = total), which
 // also clears the counts; bsum holds scan_tiles(m) + 1 words.
 void launch_scan(const Launch &L, uint32_t *counts, uint32_t m, uint32_t *bsum, uint32_t *start);
-// Provisional slots by atomic rank; lists the buckets of more than
-// kRankDirectMax particles in segs (nsegs[0] of them).  counts, m: as scanned.
+// Provisional slots by atomic rank; then every bucket of more than
+// kRankDirectMax particles is sorted by id in place (its segment listed in
+// segs, nsegs[0] of them; tmp: one uint2 per pool slot, scratch).
 void launch_scatter(const Launch &L, const PoolView &pv, const float4 *P, const uint32_t *keys, const uint32_t *ranks,
                     const uint32_t *start, uint32_t *slot_src, uint32_t *slot_id, uint4 *segs, uint32_t *nsegs,
-                    uint32_t *counts, uint32_t m);
+                    uint2 *tmp);
 // Copies positions and velocities to cell order; order[f] receives the state
 // slot of the particle in slot f (acceleration and low position words stay
-// in the state arrays, read there by the force pass).  The listed buckets are
-// sorted by id in place on the way (tmp: one uint2 per pool slot, scratch).
-void launch_gather(const Launch &L, const PoolView &pv, uint32_t *slot_src, uint32_t *slot_id, const uint32_t *keys,
-                   const uint32_t *start, const float4 *P, const float4 *V, float4 *Ps, float4 *Vs, uint32_t *order,
-                   float *soa, uint32_t *moves, const uint4 *segs, const uint32_t *nsegs, uint2 *tmp);
+// in the state arrays, read there by the force pass).
+void launch_gather(const Launch &L, const PoolView &pv, const uint32_t *slot_src, const uint32_t *slot_id,
+                   const uint32_t *keys, const uint32_t *start, const float4 *P, const float4 *V, float4 *Ps,
+                   float4 *Vs, uint32_t *order, float *soa, uint32_t *moves);
 // Writes one set of neighbour masks, MS: the slots within the substep's
 // skin radius (at least h), which the normals and forces passes walk
 // (re-testing r <= h) and XSPH walks after the move.

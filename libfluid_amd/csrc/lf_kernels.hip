@@ -45,8 +45,7 @@ namespace lf {
 // The value returned by the count atomic is the particle's provisional rank
 // inside its bucket.  Particles arrive in the previous cell order, so runs of
 // lanes share a bucket: each run issues one atomic for its length and hands
-// out consecutive ranks.  Counts are zeroed by the previous substep's scan
-// or scatter.
+// out consecutive ranks.  Counts are zeroed by the previous substep's scan.
 // Each thread takes kHashItems particles, kBlock slots apart, whose loads
 // and count atomics are issued together (the pass is latency bound).
 constexpr int kHashItems = 2;
@@ -203,52 +202,6 @@ __global__ __launch_bounds__(kBlock) void k_scan_down(uint32_t *__restrict__ cou
     if (blockIdx.x == nb - 1u && threadIdx.x == 0) start[m] = prefix + tot;
 }
 
-// The scan of at most kScanOneTiles tiles of kScanOneTile buckets in one
-// launch: each workgroup adds up the counts of every tile before its own
-// (eight 16-byte loads in flight per thread) instead of waiting for a first
-// launch to do so.  The counts are cleared by k_scatter, as other workgroups
-// still read them here.
-constexpr int kScanOneThreads = 1024;
-constexpr uint32_t kScanOneTile = 4u * kScanOneThreads, kScanOneTiles = 24u;
-__global__ __launch_bounds__(kScanOneThreads) void k_scan_one(const uint32_t *__restrict__ counts, uint32_t m,
-                                                              uint32_t *__restrict__ start) {
-    __shared__ uint32_t before_w[kScanOneThreads / 64], own_w[kScanOneThreads / 64];
-    const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
-    const uint32_t base = blockIdx.x * kScanOneTile + 4u * t;
-    const uint4 v = scan_load(counts, base, m);
-    uint32_t before = 0u;
-    for (uint32_t k0 = 0u; k0 < blockIdx.x; k0 += 8u) {  // tiles before this one: all whole
-        uint4 x[8];
-#pragma unroll
-        for (uint32_t k = 0u; k < 8u; ++k) {
-            const uint32_t tile = k0 + k < blockIdx.x ? k0 + k : 0u;
-            x[k] = *reinterpret_cast<const uint4 *>(counts + tile * kScanOneTile + 4u * t);
-        }
-#pragma unroll
-        for (uint32_t k = 0u; k < 8u; ++k)
-            if (k0 + k < blockIdx.x) before += x[k].x + x[k].y + x[k].z + x[k].w;
-    }
-    const uint32_t own = v.x + v.y + v.z + v.w;
-    const uint32_t incl = wave_incl_scan(own), all = wave_incl_scan(before);
-    if (lane == 63u) {
-        own_w[w] = incl;
-        before_w[w] = all;
-    }
-    __syncthreads();
-    uint32_t run = incl - own, total = 0u;
-#pragma unroll
-    for (uint32_t k = 0u; k < kScanOneThreads / 64; ++k) {
-        run += before_w[k] + (k < w ? own_w[k] : 0u);
-        total += before_w[k] + own_w[k];
-    }
-    const uint32_t sv[4] = {run, run + v.x, run + v.x + v.y, run + v.x + v.y + v.z};
-    if (base + 4u <= m)
-        *reinterpret_cast<uint4 *>(start + base) = make_uint4(sv[0], sv[1], sv[2], sv[3]);
-    else
-        for (uint32_t k = 0u; k < 4u && base + k < m; ++k) start[base + k] = sv[k];
-    if (blockIdx.x == gridDim.x - 1u && t == 0u) start[m] = total;
-}
-
 // ---------------------------------------------------------------------------
 // Slot of the first particle of pool bucket b of scene c:
 //   first + (start[b] - start[cell_base]) = start[b] + shift.
@@ -258,130 +211,109 @@ __device__ __forceinline__ uint32_t slot_shift(const Consts &c, const uint32_t *
 
 // 3b. segments (buckets of more than kRankDirectMax particles) sorted by id
 // in place: (slot_id, slot_src) of slots [lo, lo + size), by one workgroup of
-// NT threads: an LSD radix sort by 8 bits of the id per pass, through tmp
-// (same slots) and back.  A pass counts the digits, then places the segment
-// tile by tile (NT * kSegItems elements, each wave a run of consecutive
-// ones): a member's new place is the digit's running base, plus that digit's
-// count in the tile's earlier waves, plus its count in the wave's earlier
-// rounds, plus its rank among the earlier lanes with the same digit (lanes
-// matched by eight ballots), so every pass is stable.  Ids are unique within
-// a scene.
-constexpr int kSegItems = 4;
+// NT threads, segment after segment (k_sort_segments, after k_scatter): an LSD radix sort by 8 bits of the id
+// per pass, through tmp (same slots) and back.  A pass counts the digits,
+// then places the segment tile by tile (NT elements, in slot order): a
+// member's new place is the digit's running base, plus that digit's count
+// in the tile's earlier waves, plus its rank among the earlier lanes of its
+// wave with the same digit (lanes matched by eight ballots), so every pass
+// is stable.  Ids are unique within a scene.
 __device__ __forceinline__ uint32_t seg_digit(uint32_t id, uint32_t shift) { return (id >> shift) & 0xFFu; }
-
-// Orders a wave's LDS accesses of different lanes.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
 
 template <int NT>
 struct SegSortLds {
-    uint32_t base[256];           // running start of each digit in the destination
-    uint32_t wcnt[NT / 64][256];  // per wave: digit counts, then their prefix over waves
+    uint32_t base[256];               // running start of each digit in the destination
+    uint32_t wcnt[NT / 64][256];      // per wave: digit counts, then their prefix over waves
     uint32_t scan_tot[4];
 };
 
 template <int NT>
-__device__ void sort_segment(SegSortLds<NT> &sh, uint4 g, uint32_t *__restrict__ slot_id,
-                             uint32_t *__restrict__ slot_src, uint2 *__restrict__ tmp) {
+__device__ void sort_segments(SegSortLds<NT> &sh, const uint4 *__restrict__ segs, uint32_t nseg,
+                              uint32_t *__restrict__ slot_id, uint32_t *__restrict__ slot_src,
+                              uint2 *__restrict__ tmp) {
     static_assert(NT >= 256 && NT % 64 == 0, "the digit scan needs four waves");
     constexpr int kWaves = NT / 64;
     const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
     const uint64_t below = (1ull << lane) - 1ull;
-    const uint32_t lo = g.x, n = g.y, passes = (g.z + 7u) / 8u;
-    for (uint32_t p = 0; p < passes; ++p) {
-        const bool from_tmp = (p & 1u) != 0u;
-        const uint32_t shift = 8u * p;
-        const auto id_at = [&](uint32_t k) { return from_tmp ? tmp[lo + k].x : slot_id[lo + k]; };
-        if (t < 256u) sh.base[t] = 0u;
-        __syncthreads();
-        for (uint32_t k0 = t; k0 < n; k0 += NT * kSegItems) {  // kSegItems loads in flight
-            uint32_t id[kSegItems];
-#pragma unroll
-            for (int q = 0; q < kSegItems; ++q) {
-                const uint32_t k = k0 + (uint32_t)(q * NT);
-                id[q] = id_at(k < n ? k : k0);
-            }
-#pragma unroll
-            for (int q = 0; q < kSegItems; ++q)
-                if (k0 + (uint32_t)(q * NT) < n) atomicAdd(&sh.base[seg_digit(id[q], shift)], 1u);
-        }
-        __syncthreads();
-        // exclusive scan of the 256 digit counts (waves 0-3)
-        uint32_t v = 0u, incl = 0u;
-        if (t < 256u) {
-            v = sh.base[t];
-            incl = wave_incl_scan(v);
-            if (lane == 63u) sh.scan_tot[w] = incl;
-        }
-        __syncthreads();
-        if (t < 256u) {
-            uint32_t off = 0u;
-            for (uint32_t q = 0; q < w; ++q) off += sh.scan_tot[q];
-            sh.base[t] = off + incl - v;
-        }
-        for (uint32_t tile = 0; tile < n; tile += NT * kSegItems) {
-            __syncthreads();  // base and the last tile's counts are done with
-            for (uint32_t q = t; q < kWaves * 256u; q += NT) (&sh.wcnt[0][0])[q] = 0u;
-            uint2 e[kSegItems];
-            uint32_t d[kSegItems], rank[kSegItems];
-            const uint32_t k0 = tile + w * (64u * kSegItems) + lane;
-#pragma unroll
-            for (int q = 0; q < kSegItems; ++q) {
-                const uint32_t k = k0 + 64u * (uint32_t)q;
-                e[q] = make_uint2(0u, 0u);
-                if (k < n) e[q] = from_tmp ? tmp[lo + k] : make_uint2(slot_id[lo + k], slot_src[lo + k]);
+    for (uint32_t sg = 0; sg < nseg; ++sg) {
+        const uint4 g = segs[sg];
+        const uint32_t lo = g.x, n = g.y, passes = (g.z + 7u) / 8u;
+        for (uint32_t p = 0; p < passes; ++p) {
+            const bool from_tmp = (p & 1u) != 0u;
+            const uint32_t shift = 8u * p;
+            if (t < 256u) sh.base[t] = 0u;
+            __syncthreads();
+            for (uint32_t k = t; k < n; k += NT) {
+                const uint32_t id = from_tmp ? tmp[lo + k].x : slot_id[lo + k];
+                atomicAdd(&sh.base[seg_digit(id, shift)], 1u);
             }
             __syncthreads();
+            // exclusive scan of the 256 digit counts (waves 0-3)
+            uint32_t v = 0u, incl = 0u;
+            if (t < 256u) {
+                v = sh.base[t];
+                incl = v;
 #pragma unroll
-            for (int q = 0; q < kSegItems; ++q) {
-                const bool valid = k0 + 64u * (uint32_t)q < n;
-                d[q] = seg_digit(e[q].x, shift);
+                for (int o = 1; o < 64; o <<= 1) {
+                    const uint32_t u = __shfl_up(incl, o, 64);
+                    if ((int)lane >= o) incl += u;
+                }
+                if (lane == 63u) sh.scan_tot[w] = incl;
+            }
+            __syncthreads();
+            if (t < 256u) {
+                uint32_t off = 0u;
+                for (uint32_t q = 0; q < w; ++q) off += sh.scan_tot[q];
+                sh.base[t] = off + incl - v;
+            }
+            __syncthreads();
+            for (uint32_t tile = 0; tile < n; tile += NT) {
+                for (uint32_t q = t; q < kWaves * 256u; q += NT) (&sh.wcnt[0][0])[q] = 0u;
+                __syncthreads();
+                const uint32_t k = tile + t;
+                const bool valid = k < n;
+                uint2 e = make_uint2(0u, 0u);
+                if (valid) e = from_tmp ? tmp[lo + k] : make_uint2(slot_id[lo + k], slot_src[lo + k]);
+                const uint32_t d = seg_digit(e.x, shift);
                 uint64_t peers = __ballot(valid);
 #pragma unroll
                 for (uint32_t bit = 0; bit < 8u; ++bit) {
-                    const bool on = ((d[q] >> bit) & 1u) != 0u;
+                    const bool on = ((d >> bit) & 1u) != 0u;
                     const uint64_t m = __ballot(on);
                     peers &= on ? m : ~m;
                 }
-                const uint32_t before = (uint32_t)__popcll(peers & below), seen = sh.wcnt[w][d[q]];
-                rank[q] = seen + before;
-                wave_lds_sync();  // every lane has read its digit's count
-                if (valid && before == 0u) sh.wcnt[w][d[q]] = seen + (uint32_t)__popcll(peers);
-                wave_lds_sync();
-            }
-            __syncthreads();
-            uint32_t tile_total = 0u;
-            if (t < 256u) {  // prefix of digit t's counts over the waves
-                for (uint32_t q = 0; q < (uint32_t)kWaves; ++q) {
-                    const uint32_t c = sh.wcnt[q][t];
-                    sh.wcnt[q][t] = tile_total;
-                    tile_total += c;
+                const uint32_t rank = (uint32_t)__popcll(peers & below);
+                if (valid && rank == 0u) sh.wcnt[w][d] = (uint32_t)__popcll(peers);
+                __syncthreads();
+                uint32_t tile_total = 0u;
+                if (t < 256u) {  // prefix of digit t's counts over the waves
+                    for (uint32_t q = 0; q < (uint32_t)kWaves; ++q) {
+                        const uint32_t c = sh.wcnt[q][t];
+                        sh.wcnt[q][t] = tile_total;
+                        tile_total += c;
+                    }
                 }
-            }
-            __syncthreads();
-#pragma unroll
-            for (int q = 0; q < kSegItems; ++q) {
-                if (k0 + 64u * (uint32_t)q >= n) continue;
-                const uint32_t dst = lo + sh.base[d[q]] + sh.wcnt[w][d[q]] + rank[q];
-                if (from_tmp) {
-                    slot_id[dst] = e[q].x;
-                    slot_src[dst] = e[q].y;
-                } else {
-                    tmp[dst] = e[q];
+                __syncthreads();
+                if (valid) {
+                    const uint32_t dst = lo + sh.base[d] + sh.wcnt[w][d] + rank;
+                    if (from_tmp) {
+                        slot_id[dst] = e.x;
+                        slot_src[dst] = e.y;
+                    } else {
+                        tmp[dst] = e;
+                    }
                 }
+                __syncthreads();
+                if (t < 256u) sh.base[t] += tile_total;
+                __syncthreads();
             }
-            __syncthreads();
-            if (t < 256u) sh.base[t] += tile_total;
         }
-        __syncthreads();  // the pass's stores are visible to the next
-    }
-    if (passes & 1u) {  // the last pass wrote tmp
-        for (uint32_t k = t; k < n; k += NT) {
-            const uint2 e = tmp[lo + k];
-            slot_id[lo + k] = e.x;
-            slot_src[lo + k] = e.y;
+        if (passes & 1u) {  // the last pass wrote tmp
+            for (uint32_t k = t; k < n; k += NT) {
+                const uint2 e = tmp[lo + k];
+                slot_id[lo + k] = e.x;
+                slot_src[lo + k] = e.y;
+            }
         }
         __syncthreads();
     }
@@ -389,18 +321,14 @@ __device__ void sort_segment(SegSortLds<NT> &sh, uint4 g, uint32_t *__restrict__
 
 // 3. provisional scatter: slot = bucket start + atomic rank.  The particle
 // with rank 0 of a bucket of more than kRankDirectMax particles lists the
-// bucket's slot range as a segment for k_gather: (first slot, size, bits of
-// the scene's largest id, scene).  After a scan in one launch (k_scan_one,
-// whose workgroups read each other's counts) it clears the counts [0, clear)
-// for the next substep.
+// bucket's slot range as a segment for k_sort_segments: (first slot, size,
+// bits of the scene's largest id).
 __global__ __launch_bounds__(kBlock) void k_scatter(const Consts *__restrict__ cs, const uint32_t *__restrict__ chunk,
                                                     const float4 *__restrict__ P, const uint32_t *__restrict__ keys,
                                                     const uint32_t *__restrict__ ranks,
                                                     const uint32_t *__restrict__ start,
                                                     uint32_t *__restrict__ slot_src, uint32_t *__restrict__ slot_id,
-                                                    uint4 *__restrict__ segs, uint32_t *__restrict__ nsegs,
-                                                    uint32_t *__restrict__ counts, uint32_t clear) {
-    for (uint32_t k = blockIdx.x * kBlock + threadIdx.x; k < clear; k += gridDim.x * kBlock) counts[k] = 0u;
+                                                    uint4 *__restrict__ segs, uint32_t *__restrict__ nsegs) {
     uint32_t slot0;
     const Consts *cp = block_scene<kBlock>(cs, chunk, slot0);
     if (!cp) return;
@@ -415,76 +343,50 @@ __global__ __launch_bounds__(kBlock) void k_scatter(const Consts *__restrict__ c
         const uint32_t size = start[b + 1] - start[b];
         if (size > kRankDirectMax) {
             const uint32_t bits = cp->count > 1u ? 32u - (uint32_t)__clz(cp->count - 1u) : 1u;
-            segs[atomicAdd(nsegs, 1u)] = make_uint4(lo, size, bits, cp->scene);
+            segs[atomicAdd(nsegs, 1u)] = make_uint4(lo, size, bits, 0u);
         }
     }
+}
+
+// 3c. the listed segments, one workgroup each (grid stride over the list;
+// a workgroup with no segment exits at once).  (A ticket taken by every
+// workgroup of the scatter pass, to let its last workgroup sort, needs a
+// device-scope fence per wave, which costs far more than this launch.)
+constexpr int kSegThreads = 1024;
+constexpr int kSegBlocks = 32;
+__global__ __launch_bounds__(kSegThreads) void k_sort_segments(const uint4 *__restrict__ segs,
+                                                               const uint32_t *__restrict__ nsegs,
+                                                               uint32_t *__restrict__ slot_id,
+                                                               uint32_t *__restrict__ slot_src,
+                                                               uint2 *__restrict__ tmp) {
+    __shared__ SegSortLds<kSegThreads> sh;
+    const uint32_t nseg = *nsegs;
+    for (uint32_t sg = blockIdx.x; sg < nseg; sg += gridDim.x)
+        sort_segments<kSegThreads>(sh, segs + sg, 1u, slot_id, slot_src, tmp);
 }
 
 // 4. stable placement + payload gather (sort_by_key of Points, Velocity,
 // Acceleration, fluidsystem.cu:309-313).  The final slot of a particle is
 // its bucket start plus the number of bucket members with a smaller id, so
-// the order is (key, id) whatever order the atomics handed out.  A bucket of
-// more than kRankDirectMax particles is sorted by id in place instead, and
-// placed, by one of the launch's first kSegBlocks workgroups, which exit at
-// once where there is no such bucket (a launch of its own for them took 4.6
-// us of every substep).  Position and velocity are copied to cell order (the
-// neighbour passes gather them); the acceleration and the position's low
-// word, which only the particle's own integration reads, stay where they are:
-// order[f] records the state slot the particle in slot f came from.
-constexpr uint32_t kSegBlocks = 32;  // a multiple of 8: the other workgroups keep their XCD
+// the order is (key, id) whatever order the atomics handed out; a bucket of
+// more than kRankDirectMax particles has been sorted by id in place
+// (k_sort_segments), so there the provisional slot is the final one.  Position
+// and velocity are copied to cell order (the neighbour passes gather them);
+// the acceleration and the position's low word, which only the particle's
+// own integration reads, stay where they are: order[f] records the state
+// slot the particle in slot f came from.
 __global__ __launch_bounds__(kBlock) void k_gather(const Consts *__restrict__ cs, const uint32_t *__restrict__ chunk,
-                                                   uint32_t *__restrict__ slot_src, uint32_t *__restrict__ slot_id,
+                                                   const uint32_t *__restrict__ slot_src,
+                                                   const uint32_t *__restrict__ slot_id,
                                                    const uint32_t *__restrict__ keys,
                                                    const uint32_t *__restrict__ start, const float4 *__restrict__ P,
                                                    const float4 *__restrict__ V,
                                                    float4 *__restrict__ Ps, float4 *__restrict__ Vs,
                                                    uint32_t *__restrict__ order, float *__restrict__ soa,
                                                    uint32_t nslots, uint8_t *__restrict__ near,
-                                                   uint32_t *__restrict__ moves, const uint4 *__restrict__ segs,
-                                                   const uint32_t *__restrict__ nsegs, uint2 *__restrict__ tmp) {
-    __shared__ SegSortLds<kBlock> sh;
-    // copies the particle in state slot src to cell-order slot f
-    const auto place = [&](const Consts &c, uint32_t src, uint32_t f) -> uint32_t {
-        const float4 p = P[src], v = V[src];
-        Ps[f] = p;
-        soa[f] = p.x;
-        soa[nslots + f] = p.y;
-        soa[2 * (size_t)nslots + f] = p.z;
-        Vs[f] = v;
-        order[f] = src;
-        return skin_quantum(c, v);
-    };
-    // The scene's largest move of the substep (XSPH skin): reduced over the
-    // workgroup, then one atomicMax into the slot of the workgroup's index.
-    const auto raise = [&](uint32_t scene, uint32_t q, uint32_t k) {
-        uint32_t *wq = sh.scan_tot;
-        q = wave_max<10>(q);
-        if ((threadIdx.x & 63u) == 0u) wq[threadIdx.x >> 6] = q;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            uint32_t m = wq[0];
-#pragma unroll
-            for (int w = 1; w < kBlock / 64; ++w) m = m > wq[w] ? m : wq[w];
-            atomicMax(move_slot(moves, scene, k % kMoveSlots), m);
-        }
-    };
-    if (blockIdx.x < kSegBlocks) {
-        const uint32_t nseg = *nsegs;
-        for (uint32_t sg = blockIdx.x; sg < nseg; sg += kSegBlocks) {
-            const uint4 g = segs[sg];
-            sort_segment<kBlock>(sh, g, slot_id, slot_src, tmp);
-            uint32_t q = 0u;
-            for (uint32_t s = g.x + threadIdx.x; s < g.x + g.y; s += kBlock) {
-                const uint32_t qs = place(cs[g.w], slot_src[s], s);
-                q = q > qs ? q : qs;
-            }
-            raise(g.w, q, sg);
-            __syncthreads();
-        }
-        return;
-    }
+                                                   uint32_t *__restrict__ moves) {
     uint32_t slot0;
-    const Consts *cp = block_scene<kBlock>(cs, chunk, slot0, kSegBlocks);
+    const Consts *cp = block_scene<kBlock>(cs, chunk, slot0);
     if (!cp) return;
     const uint32_t s = slot0 + threadIdx.x;
     uint32_t q = 0u;
@@ -493,6 +395,7 @@ __global__ __launch_bounds__(kBlock) void k_gather(const Consts *__restrict__ cs
         const uint32_t b = keys[src];
         const uint32_t shift = slot_shift(*cp, start);
         const uint32_t lo = start[b] + shift, hi = start[b + 1] + shift;
+        uint32_t f = s;
         if (hi - lo <= kRankDirectMax) {
             // four members' ids loaded together per step
             uint32_t r = 0, t = lo;
@@ -501,11 +404,30 @@ __global__ __launch_bounds__(kBlock) void k_gather(const Consts *__restrict__ cs
                 r += (a0 < id ? 1u : 0u) + (a1 < id ? 1u : 0u) + (a2 < id ? 1u : 0u) + (a3 < id ? 1u : 0u);
             }
             for (; t < hi; ++t) r += (slot_id[t] < id) ? 1u : 0u;
-            q = place(*cp, src, lo + r);
+            f = lo + r;
         }
+        const float4 p = P[src], v = V[src];
+        Ps[f] = p;
+        soa[f] = p.x;
+        soa[nslots + f] = p.y;
+        soa[2 * (size_t)nslots + f] = p.z;
+        Vs[f] = v;
+        order[f] = src;
+        q = skin_quantum(*cp, v);
         if (s % kNearBlock == 0u) near[s / kNearBlock] = 0u;  // marked again by k_density
     }
-    raise(cp->scene, q, blockIdx.x);
+    // The scene's largest move of the substep (XSPH skin): reduced over the
+    // workgroup, then one atomicMax into the slot of the workgroup's index.
+    __shared__ uint32_t wq[kBlock / 64];
+    q = wave_max<10>(q);
+    if ((threadIdx.x & 63u) == 0u) wq[threadIdx.x >> 6] = q;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t m = wq[0];
+#pragma unroll
+        for (int w = 1; w < kBlock / 64; ++w) m = m > wq[w] ? m : wq[w];
+        atomicMax(move_slot(moves, cp->scene, blockIdx.x % kMoveSlots), m);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1643,6 +1565,12 @@ __device__ __forceinline__ uint32_t quad_or(uint32_t v) {
     v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true);  // lanes 2 3 0 1
     return v;
 }
+// Orders a wave's LDS accesses of different lanes (a quad is inside one wave).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // First slots and lengths of the rows q, q + 4 and (lane 0) 8 of lane q.
 struct QuadRows {
     uint32_t s[3], len[3];
@@ -2391,16 +2319,7 @@ void launch_hash(const Launch &L, const PoolView &pv, const float4 *P, uint32_t 
 
 uint32_t scan_tiles(uint32_t m) { return (m + kScanTile - 1) / kScanTile; }
 
-// Whether launch_scan scans m buckets in one launch (and launch_scatter
-// clears their counts).
-bool scan_in_one(uint32_t m) { return m <= kScanOneTiles * kScanOneTile; }
-
 void launch_scan(const Launch &L, uint32_t *counts, uint32_t m, uint32_t *bsum, uint32_t *start) {
-    if (scan_in_one(m)) {
-        LF_GO(L, k_scan_one, (m + kScanOneTile - 1u) / kScanOneTile, kScanOneThreads, L.a, L.b,
-              (const uint32_t *)counts, m, start);
-        return;
-    }
     const uint32_t nb = scan_tiles(m);
     const bool prefixed = nb > kScanDirectTiles;
     LF_GO(L, k_scan_sum, nb, kBlock, L.a, nullptr, (const uint32_t *)counts, m, bsum);
@@ -2410,16 +2329,18 @@ void launch_scan(const Launch &L, uint32_t *counts, uint32_t m, uint32_t *bsum, 
 
 void launch_scatter(const Launch &L, const PoolView &pv, const float4 *P, const uint32_t *keys, const uint32_t *ranks,
                     const uint32_t *start, uint32_t *slot_src, uint32_t *slot_id, uint4 *segs, uint32_t *nsegs,
-                    uint32_t *counts, uint32_t m) {
-    LF_GO(L, k_scatter, pv.nlaunch / kBlock, kBlock, L.a, L.b, pv.cs, pv.chunk, P, keys, ranks, start, slot_src,
-          slot_id, segs, nsegs, counts, scan_in_one(m) ? m : 0u);
+                    uint2 *tmp) {
+    LF_GO(L, k_scatter, pv.nlaunch / kBlock, kBlock, L.a, nullptr, pv.cs, pv.chunk, P, keys, ranks, start, slot_src,
+          slot_id, segs, nsegs);
+    LF_GO(L, k_sort_segments, kSegBlocks, kSegThreads, nullptr, L.b, (const uint4 *)segs, (const uint32_t *)nsegs,
+          slot_id, slot_src, tmp);
 }
 
-void launch_gather(const Launch &L, const PoolView &pv, uint32_t *slot_src, uint32_t *slot_id, const uint32_t *keys,
-                   const uint32_t *start, const float4 *P, const float4 *V, float4 *Ps, float4 *Vs, uint32_t *order,
-                   float *soa, uint32_t *moves, const uint4 *segs, const uint32_t *nsegs, uint2 *tmp) {
-    LF_GO(L, k_gather, kSegBlocks + pv.nlaunch / kBlock, kBlock, L.a, L.b, pv.cs, pv.chunk, slot_src, slot_id, keys,
-          start, P, V, Ps, Vs, order, soa, pv.nslots, pv.near, moves, segs, nsegs, tmp);
+void launch_gather(const Launch &L, const PoolView &pv, const uint32_t *slot_src, const uint32_t *slot_id,
+                   const uint32_t *keys, const uint32_t *start, const float4 *P, const float4 *V, float4 *Ps,
+                   float4 *Vs, uint32_t *order, float *soa, uint32_t *moves) {
+    LF_GO(L, k_gather, pv.nlaunch / kBlock, kBlock, L.a, L.b, pv.cs, pv.chunk, slot_src, slot_id, keys, start, P, V,
+          Ps, Vs, order, soa, pv.nslots, pv.near, moves);
 }
 
 void launch_density(const Launch &L, const PoolView &pv, int bs, const float4 *Ps, const float *soa,
