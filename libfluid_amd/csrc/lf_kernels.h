@@ -43,10 +43,11 @@ void launch_hash(const Launch &L, const PoolView &pv, const float4 *P, uint32_t 
 void launch_scan(const Launch &L, uint32_t *counts, uint32_t m, uint32_t *bsum, uint32_t *start);
 // Provisional slots by atomic rank; then every bucket of more than
 // kRankDirectMax particles is sorted by id in place (its segment listed in
-// segs, nsegs[0] of them; tmp: one uint2 per pool slot, scratch).
+// segs, nsegs[0] of them; tmp: one uint2 per pool slot, scratch).  counts, m:
+// as scanned.
 void launch_scatter(const Launch &L, const PoolView &pv, const float4 *P, const uint32_t *keys, const uint32_t *ranks,
                     const uint32_t *start, uint32_t *slot_src, uint32_t *slot_id, uint4 *segs, uint32_t *nsegs,
-                    uint2 *tmp);
+                    uint2 *tmp, uint32_t *counts, uint32_t m);
 // Copies positions and velocities to cell order; order[f] receives the state
 // slot of the particle in slot f (acceleration and low position words stay
 // in the state arrays, read there by the force pass).

@@ -206,7 +206,8 @@ extern "C" int lf_step_noalloc(const lf_params *p, uint32_t num_particles, float
         // One substep, the pool's sequence (Pool::enqueue_sort, enqueue_substep).
         launch_hash(L, pv, b.P0, b.keys, b.ranks, b.counts, b.flags, b.moves, b.nsegs);
         launch_scan(L, b.counts, buckets, b.bsum, b.start);
-        launch_scatter(L, pv, b.P0, b.keys, b.ranks, b.start, b.slot_src, b.slot_id, b.segs, b.nsegs, b.segtmp);
+        launch_scatter(L, pv, b.P0, b.keys, b.ranks, b.start, b.slot_src, b.slot_id, b.segs, b.nsegs, b.segtmp,
+                       b.counts, buckets);
         launch_gather(L, pv, b.slot_src, b.slot_id, b.keys, b.start, b.P0, b.V0, b.P1, b.V1, b.ranks, b.soa, b.moves);
         launch_density(L, pv, t.density, b.P1, b.soa, b.start, b.D, b.Q, b.Pr, b.MS, b.flags, b.moves);
         if (!c.lazy_normal)
