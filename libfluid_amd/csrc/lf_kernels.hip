@@ -1221,7 +1221,17 @@ __device__ __forceinline__ bool pair_term(const Consts &c, const PairSelf &me, c
     const float inv_r = frsq(rr);
     const float r = rr * inv_r;
     const float irj = q.w;
-    float hr = fmaxf(c.h - r, 0.0f);
+    // h - r in one rounding with r's product, except in the near-isolated walk
+    // (written out: left to the compiler, the choice changes with the code
+    // around it).
+    float hr;
+    if constexpr (F) {
+#pragma clang fp contract(off)
+        const float d = c.h - r;
+        hr = fmaxf(d, 0.0f);
+    } else {
+        hr = fmaxf(__builtin_fmaf(-rr, inv_r, c.h), 0.0f);
+    }
     t.frag = false;
     double hrd = 0.0;
     if constexpr (F) {
