@@ -2027,14 +2027,22 @@ __global__ __launch_bounds__(kQuadBlock) void k_forces_quad(
     if (!cp) return;
     const Consts &c = *cp;
     const uint32_t move_q = scene_move_q(moves, c.scene);
-    if (i >= c.first + c.count) return;
     const uint32_t *st = start + c.cell_base;
     const uint32_t shift = c.first - st[0];
-    const float4 pi = Ps[i], vi = Vs[i], di = D[i];
+    const bool live = i < c.first + c.count, in_grid = live && i < st[c.ncells] + shift;
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 pi = live ? Ps[i] : zero, vi = live ? Vs[i] : zero, di = live ? D[i] : zero;
+    QuadRows rows = {};
+    if (in_grid) rows = quad_rows(c, st, shift, pi, q);
+    // The near-isolated walk rounds an ordinary pair's h - r differently
+    // (pair_term), so it is chosen for the same 64 slots as in k_forces, the
+    // workgroup's.
+    bool fragile = false;
+    if (flag_set(flag_word(flags, c.scene), kFragileByte)) fragile = __syncthreads_or(quad_near(near, rows)) != 0;
+    if (!live) return;
     Forces f;
-    if (i < st[c.ncells] + shift) {
-        const PairSelf me{pi, vi, di, c.has_tension ? N[i] : make_float4(0.f, 0.f, 0.f, 0.f), di.w * di.w};
-        const QuadRows rows = quad_rows(c, st, shift, pi, q);
+    if (in_grid) {
+        const PairSelf me{pi, vi, di, c.has_tension ? N[i] : zero, di.w * di.w};
         const RowSource src{c, st, shift, Ps, soa, moves, nullptr};
         PairSums sum;
         auto walk = [&]<bool V, bool T, bool F>() {
@@ -2062,7 +2070,7 @@ __global__ __launch_bounds__(kQuadBlock) void k_forces_quad(
                     walk.template operator()<false, false, F>();
             }
         };
-        if (flag_set(flag_word(flags, c.scene), kFragileByte) && lanes(quad_near(near, rows)))
+        if (fragile)
             terms.template operator()<true>();
         else
             terms.template operator()<false>();
