@@ -94,6 +94,19 @@ void launch_carry(hipStream_t st, uint32_t first, uint32_t count, const float4 *
                   float4 *L2);
 void launch_export(hipStream_t st, const Consts &c, const float4 *P, const float4 *V, const float4 *A,
                    const float4 *D, bool by_id, float *out, uint32_t *ids);
+// As launch_upload / launch_export with one float3 array per quantity; null
+// ones are taken as zero / left out.
+void launch_upload_planes(hipStream_t st, const float *pos, const float *vel, const float *acc, uint32_t first,
+                          uint32_t id0, uint32_t count, float4 *P, float4 *V, float4 *A, float4 *Lw);
+void launch_export_planes(hipStream_t st, const Consts &c, const float4 *P, const float4 *V, const float4 *A,
+                          const float4 *D, bool by_id, float *pos, float *col, float *vel, float *acc, uint32_t *ids);
+constexpr uint32_t kCopySpans = 5;
+struct CopySpans {
+    const void *src[kCopySpans];
+    void *dst[kCopySpans];
+    size_t bytes[kCopySpans];
+};
+void launch_copy_spans(hipStream_t st, const CopySpans &c, uint32_t count);
 // Exact state (12 floats per particle: P.xyz, L.xyz, V.xyz, A.xyz), id order.
 void launch_state_out(hipStream_t st, const Consts &c, const float4 *P, const float4 *Lw, const float4 *V,
                       const float4 *A, float *out);

@@ -2136,6 +2136,22 @@ __global__ __launch_bounds__(kBlock) void k_upload(const float *__restrict__ sta
     L[slot] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 }
 
+// The same from one float3 array per quantity (vel and acc may be null: zero).
+__global__ __launch_bounds__(kBlock) void k_upload_planes(const float *__restrict__ pos, const float *__restrict__ vel,
+                                                          const float *__restrict__ acc, uint32_t first, uint32_t id0,
+                                                          uint32_t count, float4 *__restrict__ P,
+                                                          float4 *__restrict__ V, float4 *__restrict__ A,
+                                                          float4 *__restrict__ L) {
+    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+    if (k >= count) return;
+    const size_t o = 3 * (size_t)k;
+    const uint32_t id = id0 + k, slot = first + id;
+    P[slot] = make_float4(pos[o], pos[o + 1], pos[o + 2], __uint_as_float(id));
+    V[slot] = vel ? make_float4(vel[o], vel[o + 1], vel[o + 2], 0.0f) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    A[slot] = acc ? make_float4(acc[o], acc[o + 1], acc[o + 2], 0.0f) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    L[slot] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+}
+
 __global__ __launch_bounds__(kBlock) void k_init_state(uint32_t first, uint32_t count, float4 *__restrict__ P,
                                                        float4 *__restrict__ V, float4 *__restrict__ A,
                                                        float4 *__restrict__ L, float4 *__restrict__ D) {
@@ -2216,6 +2232,56 @@ __global__ __launch_bounds__(kBlock) void k_export(Consts c, const float4 *__res
     o[6] = v.x; o[7] = v.y; o[8] = v.z;
     o[9] = a.x; o[10] = a.y; o[11] = a.z;
     ids[dst] = id;
+}
+
+// The same as one float3 array per quantity, those that are not null.
+__global__ __launch_bounds__(kBlock) void k_export_planes(Consts c, const float4 *__restrict__ P,
+                                                          const float4 *__restrict__ V, const float4 *__restrict__ A,
+                                                          const float4 *__restrict__ D, int by_id,
+                                                          float *__restrict__ pos, float *__restrict__ col,
+                                                          float *__restrict__ vel, float *__restrict__ acc,
+                                                          uint32_t *__restrict__ ids) {
+    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+    if (k >= c.count) return;
+    const uint32_t s = c.first + k;
+    const float4 p = P[s];
+    const uint32_t id = __float_as_uint(p.w);
+    const uint32_t dst = by_id ? id : k;
+    const auto put = [&](float *out, float x, float y, float z) {
+        float *o = out + 3 * (size_t)dst;
+        o[0] = x;
+        o[1] = y;
+        o[2] = z;
+    };
+    if (pos) put(pos, p.x, p.y, p.z);
+    if (col) {
+        const float3 rgb = density_colour(c, D[s].x);
+        put(col, rgb.x, rgb.y, rgb.z);
+    }
+    if (vel) {
+        const float4 v = V[s];
+        put(vel, v.x, v.y, v.z);
+    }
+    if (acc) {
+        const float4 a = A[s];
+        put(acc, a.x, a.y, a.z);
+    }
+    if (ids) ids[dst] = id;
+}
+
+// Copies up to kCopySpans spans (16-byte aligned, whole words) in one launch:
+// between device memory and pinned host memory, where a few hundred kilobytes
+// would spend longer in the set-up of one DMA per span.
+__global__ __launch_bounds__(kBlock) void k_copy_spans(CopySpans c) {
+    const uint32_t *__restrict__ src = static_cast<const uint32_t *>(c.src[blockIdx.y]);
+    uint32_t *__restrict__ dst = static_cast<uint32_t *>(c.dst[blockIdx.y]);
+    const size_t words = c.bytes[blockIdx.y] / 4u;
+    const size_t k = 4u * ((size_t)blockIdx.x * kBlock + threadIdx.x);
+    if (k + 4u <= words) {
+        *reinterpret_cast<uint4 *>(dst + k) = *reinterpret_cast<const uint4 *>(src + k);
+    } else {
+        for (size_t q = k; q < words; ++q) dst[q] = src[q];
+    }
 }
 
 // Exact state in particle-id order, 12 floats per particle: position high
@@ -2520,6 +2586,28 @@ void launch_export(hipStream_t st, const Consts &c, const float4 *P, const float
     if (c.count)
         hipLaunchKernelGGL(k_export, dim3(blocks_for(c.count)), dim3(kBlock), 0, st, c, P, V, A, D, by_id ? 1 : 0,
                            out, ids);
+}
+
+void launch_upload_planes(hipStream_t st, const float *pos, const float *vel, const float *acc, uint32_t first,
+                          uint32_t id0, uint32_t count, float4 *P, float4 *V, float4 *A, float4 *Lw) {
+    if (count)
+        hipLaunchKernelGGL(k_upload_planes, dim3(blocks_for(count)), dim3(kBlock), 0, st, pos, vel, acc, first, id0,
+                           count, P, V, A, Lw);
+}
+
+void launch_export_planes(hipStream_t st, const Consts &c, const float4 *P, const float4 *V, const float4 *A,
+                          const float4 *D, bool by_id, float *pos, float *col, float *vel, float *acc,
+                          uint32_t *ids) {
+    if (c.count)
+        hipLaunchKernelGGL(k_export_planes, dim3(blocks_for(c.count)), dim3(kBlock), 0, st, c, P, V, A, D,
+                           by_id ? 1 : 0, pos, col, vel, acc, ids);
+}
+
+void launch_copy_spans(hipStream_t st, const CopySpans &c, uint32_t count) {
+    size_t most = 0;
+    for (uint32_t k = 0; k < count; ++k) most = std::max(most, c.bytes[k]);
+    if (most)
+        hipLaunchKernelGGL(k_copy_spans, dim3(blocks_for((most + 15) / 16), count), dim3(kBlock), 0, st, c);
 }
 
 void launch_state_out(hipStream_t st, const Consts &c, const float4 *P, const float4 *Lw, const float4 *V,

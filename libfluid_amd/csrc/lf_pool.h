@@ -127,6 +127,14 @@ class Pool {
     };
     template <class T>
     int dalloc(T **p, size_t count);
+    // Copies between device and the caller's (pageable) memory through pinned
+    // staging, to the host after what the stream holds; returns when done.
+    struct Span {
+        char *dev, *host;
+        size_t bytes;
+    };
+    int copy_spans(const std::vector<Span> &spans, bool to_host);
+    bool stage(int k);
     void release();
     Consts make_scene_consts(uint32_t id) const;
     int push_tables();
@@ -191,6 +199,13 @@ class Pool {
     hipEvent_t tables_ev_[kTableRing] = {};
     bool tables_ev_pending_[kTableRing] = {};
     int table_slot_ = 0;
+
+    // Pinned staging of uploads and downloads, a buffer and an event per
+    // copying thread: made when first needed, kept until release().
+    static constexpr int kStages = 8;
+    static constexpr size_t kStageBytes = size_t(2) << 20;
+    char *stage_[kStages] = {};
+    hipEvent_t stage_ev_[kStages] = {};
 
     // captured substep, one per pairing of the state and scratch A/L buffers
     hipGraph_t graph_[2] = {};

@@ -14,6 +14,7 @@
 #include <cstring>
 #include <atomic>
 #include <numeric>
+#include <thread>
 
 #include "lf_internal.h"
 
@@ -182,6 +183,12 @@ void Pool::release() {
         pin_chunk_[k] = nullptr;
         tables_ev_[k] = nullptr;
         tables_ev_pending_[k] = false;
+    }
+    for (int k = 0; k < kStages; ++k) {
+        if (stage_[k]) (void)hipHostFree(stage_[k]);
+        if (stage_ev_[k]) (void)hipEventDestroy(stage_ev_[k]);
+        stage_[k] = nullptr;
+        stage_ev_[k] = nullptr;
     }
     if (stream_) (void)hipStreamDestroy(stream_);
     stream_ = nullptr;
@@ -706,23 +713,16 @@ int Pool::upload(uint32_t id, uint32_t first, uint32_t count, const float *pos, 
                     (unsigned long long)first + count, s->n);
     if (count == 0) return LF_OK;
     if (int rc = to_id_order(id)) return rc;
-    std::vector<float> stage(9 * (size_t)count, 0.0f);
-    for (size_t k = 0; k < count; ++k)
-        for (int a = 0; a < 3; ++a) {
-            stage[9 * k + a] = pos[3 * k + a];
-            if (vel) stage[9 * k + 3 + a] = vel[3 * k + a];
-            if (acc) stage[9 * k + 6 + a] = acc[3 * k + a];
-        }
-    float *d_stage = nullptr;
-    if (int rc = dalloc(&d_stage, stage.size())) return rc;
-    hipError_t e = hipMemcpyAsync(d_stage, stage.data(), stage.size() * sizeof(float), hipMemcpyHostToDevice, stream_);
-    if (e == hipSuccess) {
-        launch_upload(stream_, d_stage, s->first, first, count, P0_, V0_, A0_, L0_);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = hipStreamSynchronize(stream_);
-    dev_free(d_stage);
-    if (e != hipSuccess) return fail(LF_ERR_HIP, "upload: %s", hipGetErrorString(e));
+    // Through A1, L1 and V1, which hold nothing between substeps.
+    const size_t bytes = 12 * (size_t)count;
+    std::vector<Span> spans{{(char *)A1_, (char *)pos, bytes}};
+    if (vel) spans.push_back({(char *)L1_, (char *)vel, bytes});
+    if (acc) spans.push_back({(char *)V1_, (char *)acc, bytes});
+    if (int rc = copy_spans(spans, false)) return rc;
+    launch_upload_planes(stream_, (const float *)A1_, vel ? (const float *)L1_ : nullptr,
+                         acc ? (const float *)V1_ : nullptr, s->first, first, count, P0_, V0_, A0_, L0_);
+    if (int rc = check_launch("upload")) return rc;
+    LF_HIP(hipStreamSynchronize(stream_));
     return LF_OK;
 }
 
@@ -745,34 +745,137 @@ int Pool::download(uint32_t id, int order, float *pos, float *col, float *vel, f
     if (!s) return fail(LF_ERR_INVALID, "download: no scene %u", id);
     if (order != LF_ORDER_CELL && order != LF_ORDER_ID) return fail(LF_ERR_INVALID, "download: bad order %d", order);
     const Consts c = make_scene_consts(id);
-    const size_t n = s->n;
-    float *d_out = nullptr;
-    uint32_t *d_ids = nullptr;
-    if (int rc = dalloc(&d_out, 12 * n)) return rc;
-    if (int rc = dalloc(&d_ids, n)) {
-        dev_free(d_out);
-        return rc;
-    }
-    launch_export(stream_, c, P0_, V0_, A0_, D_, order == LF_ORDER_ID, d_out, d_ids);
-    hipError_t e = hipGetLastError();
-    std::vector<float> host(12 * n);
-    std::vector<uint32_t> hid(n);
-    if (e == hipSuccess) e = hipMemcpyAsync(host.data(), d_out, host.size() * sizeof(float), hipMemcpyDeviceToHost, stream_);
-    if (e == hipSuccess) e = hipMemcpyAsync(hid.data(), d_ids, hid.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, stream_);
-    if (e == hipSuccess) e = hipStreamSynchronize(stream_);
-    dev_free(d_out);
-    dev_free(d_ids);
-    if (e != hipSuccess) return fail(LF_ERR_HIP, "download: %s", hipGetErrorString(e));
-    for (size_t k = 0; k < n; ++k) {
-        const float *h = &host[12 * k];
-        for (int a = 0; a < 3; ++a) {
-            if (pos) pos[3 * k + a] = h[a];
-            if (col) col[3 * k + a] = h[3 + a];
-            if (vel) vel[3 * k + a] = h[6 + a];
-            if (acc) acc[3 * k + a] = h[9 + a];
+    // The arrays asked for are laid out in A1, L1 and V1, which hold nothing
+    // between substeps (48 bytes a slot), and copied from there; in two turns
+    // where they do not all fit.
+    const size_t n = s->n, room = 16 * (size_t)nslots_;
+    struct Plane {
+        void *user;
+        size_t bytes;
+        void *dev = nullptr;
+        bool done = false;
+    };
+    Plane pl[5] = {{pos, 12 * n}, {ids, 4 * n}, {col, 12 * n}, {vel, 12 * n}, {acc, 12 * n}};
+    for (bool more = true; more;) {
+        more = false;
+        char *arena[3] = {(char *)A1_, (char *)L1_, (char *)V1_};
+        size_t used[3] = {0, 0, 0};
+        std::vector<Span> spans;
+        for (Plane &p : pl) {
+            p.dev = nullptr;
+            if (!p.user || p.done) continue;
+            for (int k = 0; k < 3 && !p.dev; ++k)
+                if (used[k] + p.bytes <= room) {
+                    p.dev = arena[k] + used[k];
+                    used[k] += (p.bytes + 15) / 16 * 16;
+                }
+            if (!p.dev) {
+                more = true;
+                continue;
+            }
+            p.done = true;
+            spans.push_back({(char *)p.dev, (char *)p.user, p.bytes});
         }
-        if (ids) ids[k] = hid[k];
+        launch_export_planes(stream_, c, P0_, V0_, A0_, D_, order == LF_ORDER_ID, (float *)pl[0].dev,
+                             (float *)pl[2].dev, (float *)pl[3].dev, (float *)pl[4].dev, (uint32_t *)pl[1].dev);
+        if (int rc = check_launch("download")) return rc;
+        if (int rc = copy_spans(spans, true)) return rc;
     }
+    return LF_OK;
+}
+
+// Makes staging buffer k; false if it cannot be had.
+bool Pool::stage(int k) {
+    if (stage_[k]) return true;
+    if (hipHostMalloc((void **)&stage_[k], kStageBytes, hipHostMallocDefault) != hipSuccess) {
+        stage_[k] = nullptr;
+        (void)hipGetLastError();
+        return false;
+    }
+    if (hipEventCreateWithFlags(&stage_ev_[k], hipEventDisableTiming) != hipSuccess) {
+        (void)hipHostFree(stage_[k]);
+        stage_[k] = nullptr;
+        stage_ev_[k] = nullptr;
+        (void)hipGetLastError();
+        return false;
+    }
+    return true;
+}
+
+// The caller's arrays are pageable, often fresh pages that the kernel has yet
+// to clear: what a large copy takes is the host's side of it.  Up to kStages
+// threads each take the next piece of at most kStageBytes through a pinned
+// buffer of their own.  Small copies go through one buffer by a kernel.
+int Pool::copy_spans(const std::vector<Span> &spans, bool to_host) {
+    size_t total = 0;
+    for (const Span &s : spans) total += (s.bytes + 15) / 16 * 16;
+    if (total == 0) {
+        if (to_host) LF_HIP(hipStreamSynchronize(stream_));
+        return LF_OK;
+    }
+    if (!stage(0)) {  // no pinned memory: plain copies
+        for (const Span &s : spans)
+            LF_HIP(hipMemcpyAsync(to_host ? s.host : s.dev, to_host ? s.dev : s.host, s.bytes,
+                                  to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, stream_));
+        LF_HIP(hipStreamSynchronize(stream_));
+        return LF_OK;
+    }
+    if (total <= kStageBytes && spans.size() <= kCopySpans) {
+        CopySpans c{};
+        size_t at = 0;
+        for (size_t k = 0; k < spans.size(); ++k) {
+            char *pin = stage_[0] + at;
+            if (!to_host) std::memcpy(pin, spans[k].host, spans[k].bytes);
+            c.src[k] = to_host ? spans[k].dev : pin;
+            c.dst[k] = to_host ? pin : spans[k].dev;
+            c.bytes[k] = spans[k].bytes;
+            at += (spans[k].bytes + 15) / 16 * 16;
+        }
+        launch_copy_spans(stream_, c, (uint32_t)spans.size());
+        if (int rc = check_launch("copy")) return rc;
+        LF_HIP(hipStreamSynchronize(stream_));
+        at = 0;
+        for (size_t k = 0; to_host && k < spans.size(); ++k) {
+            std::memcpy(spans[k].host, stage_[0] + at, spans[k].bytes);
+            at += (spans[k].bytes + 15) / 16 * 16;
+        }
+        return LF_OK;
+    }
+    std::vector<Span> pieces;
+    for (const Span &s : spans)
+        for (size_t o = 0; o < s.bytes; o += kStageBytes)
+            pieces.push_back({s.dev + o, s.host + o, std::min(kStageBytes, s.bytes - o)});
+    std::atomic<size_t> next{0};
+    std::atomic<int> error{(int)hipSuccess};
+    const auto work = [&](int w) {
+        hipError_t e = hipSetDevice(device_);
+        while (e == hipSuccess && error.load() == (int)hipSuccess) {
+            const size_t k = next.fetch_add(1);
+            if (k >= pieces.size()) break;
+            const Span &p = pieces[k];
+            if (!to_host) std::memcpy(stage_[w], p.host, p.bytes);
+            e = hipMemcpyAsync(to_host ? stage_[w] : p.dev, to_host ? p.dev : stage_[w], p.bytes,
+                               to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, stream_);
+            if (e == hipSuccess) e = hipEventRecord(stage_ev_[w], stream_);
+            if (e == hipSuccess) e = hipEventSynchronize(stage_ev_[w]);
+            if (e == hipSuccess && to_host) std::memcpy(p.host, stage_[w], p.bytes);
+        }
+        if (e != hipSuccess) error.store((int)e);
+    };
+    std::thread helpers[kStages];
+    const size_t want = std::min<size_t>(kStages, pieces.size());
+    for (size_t w = 1; w < want && stage((int)w); ++w) {
+        try {
+            helpers[w] = std::thread(work, (int)w);
+        } catch (...) {  // no more threads: the others do it
+            break;
+        }
+    }
+    work(0);
+    for (std::thread &h : helpers)
+        if (h.joinable()) h.join();
+    if (error.load() != (int)hipSuccess)
+        return fail(LF_ERR_HIP, "copy: %s", hipGetErrorString((hipError_t)error.load()));
     return LF_OK;
 }
 
