@@ -609,13 +609,16 @@ void Pool::advance_state() {
 // Launches of the executable graphs may still be queued: wait for them
 // before destroying them.
 void Pool::drop_graph() {
-    if ((graph_exec_[0] || graph_exec_[1]) && stream_) (void)hipStreamSynchronize(stream_);
-    for (int p = 0; p < 2; ++p) {
-        if (graph_exec_[p]) (void)hipGraphExecDestroy(graph_exec_[p]);
-        if (graph_[p]) (void)hipGraphDestroy(graph_[p]);
-        graph_exec_[p] = nullptr;
-        graph_[p] = nullptr;
-    }
+    bool any = false;
+    for (auto &pair : graph_exec_) any = any || pair[0] || pair[1];
+    if (any && stream_) (void)hipStreamSynchronize(stream_);
+    for (int l = 0; l < 2; ++l)
+        for (int p = 0; p < 2; ++p) {
+            if (graph_exec_[l][p]) (void)hipGraphExecDestroy(graph_exec_[l][p]);
+            if (graph_[l][p]) (void)hipGraphDestroy(graph_[l][p]);
+            graph_exec_[l][p] = nullptr;
+            graph_[l][p] = nullptr;
+        }
 }
 
 void Pool::set_graphs(bool on) {
@@ -633,17 +636,22 @@ int Pool::run_substeps(uint32_t substeps) {
         return check_launch("step");
     }
     const std::pair<uint32_t, uint32_t> span{span_slots_, span_buckets_};
-    if ((graph_exec_[0] || graph_exec_[1]) &&
+    if ((graph_exec_[0][0] || graph_exec_[0][1] || graph_exec_[1][0] || graph_exec_[1][1]) &&
         (graph_normals_ != any_separate_normals() || graph_full_ != any_full() || graph_paused_ != paused_ranges() || graph_span_ != span))
         drop_graph();
-    for (uint32_t k = 0; k < substeps; ++k) {
-        hipGraphExec_t &ge = graph_exec_[parity_];
+    for (uint32_t k = 0; k < substeps;) {
+        const int len = substeps - k >= (uint32_t)kGraphRun ? 1 : 0;
+        hipGraphExec_t &ge = graph_exec_[len][parity_];
         if (!ge) {
-            // One substep captured once per pairing of the state and scratch
-            // A/L buffers; the scene table it reads lives in device memory,
-            // so later table changes need no new capture.
+            // One substep, or kGraphRun of them, captured once per pairing of
+            // the state and scratch A/L buffers; the scene table they read
+            // lives in device memory, so later table changes need no new
+            // capture.
             LF_HIP(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
-            enqueue_substep();
+            for (int q = 0; q < (len ? kGraphRun : 1); ++q) {
+                enqueue_substep();
+                if (len) advance_state();  // an even number of times
+            }
             hipGraph_t g = nullptr;
             hipError_t e = hipStreamEndCapture(stream_, &g);
             if (e != hipSuccess) return fail(LF_ERR_HIP, "step: graph capture failed: %s", hipGetErrorString(e));
@@ -653,14 +661,19 @@ int Pool::run_substeps(uint32_t substeps) {
                 ge = nullptr;
                 return fail(LF_ERR_HIP, "step: graph instantiation failed: %s", hipGetErrorString(e));
             }
-            graph_[parity_] = g;
+            graph_[len][parity_] = g;
             graph_normals_ = any_separate_normals();
             graph_full_ = any_full();
             graph_paused_ = paused_ranges();
             graph_span_ = span;
         }
         LF_HIP(hipGraphLaunch(ge, stream_));
-        advance_state();
+        if (len) {
+            k += kGraphRun;
+        } else {
+            advance_state();
+            ++k;
+        }
     }
     return LF_OK;
 }
