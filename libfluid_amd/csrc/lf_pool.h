@@ -117,6 +117,10 @@ class Pool {
     // forces, xsph) at block size 128 << b; may be null.
     int autotune(uint32_t reps, double ms[4][3]);
     void set_graphs(bool on);
+    // Whether calls of fewer than kGraphRun substeps replay graphs too (the
+    // default).  A graph launch reaches an idle device some 8 us sooner than
+    // its kernels one by one, but leaves it idle some 6 us between two.
+    void set_short_graphs(bool on) { short_graphs_ = on; }
 
   private:
     struct Exporter;
@@ -166,7 +170,7 @@ class Pool {
     uint32_t span_slots_ = 0, span_buckets_ = 0;
     int debug_ = 0;
     Tuning tune_{};
-    bool use_graphs_ = true;
+    bool use_graphs_ = true, short_graphs_ = true;
 
     // device arrays: state (P0,V0,A0,L0) and the substep's working arrays
     float4 *P0_ = nullptr, *P1_ = nullptr, *V0_ = nullptr, *V1_ = nullptr, *V2_ = nullptr;

@@ -628,7 +628,7 @@ void Pool::set_graphs(bool on) {
 
 int Pool::run_substeps(uint32_t substeps) {
     if (int rc = push_tables()) return rc;
-    if (!use_graphs_ || prof_mask_) {
+    if (!use_graphs_ || prof_mask_ || (!short_graphs_ && substeps < (uint32_t)kGraphRun)) {
         for (uint32_t k = 0; k < substeps; ++k) {
             enqueue_substep();
             advance_state();

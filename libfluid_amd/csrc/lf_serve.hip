@@ -313,6 +313,9 @@ int lf_server_create(uint32_t max_particles, uint32_t max_cells, uint32_t max_sc
         return rc;
     }
     s->policy = policy;
+    // Ticks run ahead of the device, one substep each (40 jobs of 4,096 to
+    // 65,536 particles: 58.3 ms with a graph per tick, 53.2 without).
+    s->pool.set_short_graphs(false);
     *out = s;
     return LF_OK;
 }
