@@ -861,7 +861,8 @@ int Pool::copy_spans(const std::vector<Span> &spans, bool to_host) {
     std::atomic<size_t> next{0};
     std::atomic<int> error{(int)hipSuccess};
     const auto work = [&](int w) {
-        hipError_t e = hipSetDevice(device_);
+        // (the caller's thread keeps its own current device)
+        hipError_t e = w ? hipSetDevice(device_) : hipSuccess;
         while (e == hipSuccess && error.load() == (int)hipSuccess) {
             const size_t k = next.fetch_add(1);
             if (k >= pieces.size()) break;
