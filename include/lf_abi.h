@@ -242,7 +242,9 @@ int lf_export_wait(lf_scene *s);
  *      derived from the largest cell occupancy every substep,
  *      fluidsystem.cu:319-323) ------------------------------------------- */
 /* Workgroup sizes of the density, normals, forces and XSPH passes, each 128,
- * 256 or 512 (default 256).  Results do not depend on them. */
+ * 256 or 512 (default 256); steps of few particles take four lanes per
+ * particle in workgroups of 256 whatever is set.  Results do not depend on
+ * them. */
 int lf_set_tuning(lf_scene *s, const int block_sizes[4]);
 int lf_get_tuning(const lf_scene *s, int block_sizes[4]);
 /* Walk modes of the normals, forces and XSPH passes: 1 walks the density

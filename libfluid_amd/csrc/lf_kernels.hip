@@ -1014,8 +1014,8 @@ __global__ __launch_bounds__(BS) void k_density(const Consts *__restrict__ cs, c
     // load's address is the lane's row offset plus a scalar (buffer
     // soffset).  Each mask word is built as m = 2m + bit (a funnel shift of
     // the sign bit in), which leaves slot k at bit n-1-k of the n slots
-    // scanned into it; one bit reversal per row moves it to bit k.  Slots
-    // past 64 (rows without masks) are tested per lane.  Only the centre row
+    // scanned into it; one bit reversal per row moves it to bit k.  A row's
+    // slots past 64 follow below, 32 to a word.  Only the centre row
     // (r = 4: dz = dy = 0) holds the particle itself.
     const float nh2s = -h2s, ninv_h2 = -c.inv_h2;
     const float c1 = (c.h2 - h2s) * c.inv_h2;  // h2 - h2s is exact: h2 <= h2s <= 2 h2
