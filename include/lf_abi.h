@@ -4,6 +4,10 @@
  * Plain C: opaque handles, plain pointers and sizes, int status codes.
  * Every function returns LF_OK (0) or a negative LF_ERR_* code; the message
  * of the last failure on the calling thread is returned by lf_last_error().
+ * Handles are independent of one another.  Uploads, downloads and steps of one
+ * scene or batch may come from several threads: each runs as a whole before
+ * the next begins.  Other calls on one handle must not overlap, and a server
+ * has one caller.
  *
  * The reference (NCCA/libfluid) has no C ABI: its boundary is the C++ class
  * FluidSystem (libfluid/include/fluidsystem.h:16-126).  Each entry point

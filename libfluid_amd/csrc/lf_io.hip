@@ -30,6 +30,7 @@ namespace lf {
 // exact state
 
 int Pool::save_state(uint32_t id, std::vector<float> &out) {
+    const Scratch lock(scratch_);
     const SceneRec *s = scene(id);
     if (!s) return fail(LF_ERR_INVALID, "save_state: no scene %u", id);
     const size_t n = s->n;
@@ -46,6 +47,7 @@ int Pool::save_state(uint32_t id, std::vector<float> &out) {
 }
 
 int Pool::load_state(uint32_t id, const float *in, uint64_t steps) {
+    const Scratch lock(scratch_);
     SceneRec *s = id < scenes_.size() && scenes_[id].live ? &scenes_[id] : nullptr;
     if (!s || !in) return fail(LF_ERR_INVALID, "load_state: bad scene %u or null data", id);
     const size_t n = s->n;
@@ -70,6 +72,7 @@ int Pool::load_state(uint32_t id, const float *in, uint64_t steps) {
 
 int Pool::setup_jitter(uint32_t id, uint32_t id0, uint32_t nx, uint32_t ny, uint32_t nz, float dx, const float o[3],
                        float jitter, uint64_t seed) {
+    const Scratch lock(scratch_);
     const SceneRec *s = scene(id);
     if (!s || !o) return fail(LF_ERR_INVALID, "setup_jitter: bad scene %u or null origin", id);
     const uint64_t count = (uint64_t)nx * ny * nz;
@@ -85,6 +88,7 @@ int Pool::setup_jitter(uint32_t id, uint32_t id0, uint32_t nx, uint32_t ny, uint
 
 int Pool::setup_block(uint32_t id, uint32_t id0, uint32_t n, const float mn[3], const float mx[3], uint32_t *written,
                       float *mass, float *psize) {
+    const Scratch lock(scratch_);
     const SceneRec *s = scene(id);
     if (!s || !mn || !mx || n == 0) return fail(LF_ERR_INVALID, "setup_block: bad scene %u or arguments", id);
     if ((uint64_t)id0 + n > s->n)

@@ -10,6 +10,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <vector>
 
 #include "lf_abi.h"
@@ -159,6 +160,13 @@ class Pool {
     bool any_full() const;
     PoolView view() const { return PoolView{d_cs_, d_chunk_, nslots_, span_slots_, near_, any_full()}; }
     void set_spans();
+
+    // Held by every call that uses the scratch arrays (P1, V1, A1, L1) or the
+    // transfers' staging: a transfer lays its data out there and returns when
+    // it is across, so the next call, from another thread too, finds them
+    // free.  (Recursive: add_scene, upload and the like call one another.)
+    std::recursive_mutex scratch_;
+    using Scratch = std::lock_guard<std::recursive_mutex>;
 
     int device_ = 0;
     hipStream_t stream_ = nullptr;

@@ -407,6 +407,7 @@ int Pool::compact() {
 }
 
 int Pool::add_scene(const lf_params &p, uint32_t n, float dt, uint32_t *id) {
+    const Scratch lock(scratch_);
     if (!id) return fail(LF_ERR_INVALID, "add_scene: null id");
     if (int rc = lf_params_check(&p)) return rc;
     if (n == 0) return fail(LF_ERR_INVALID, "add_scene: zero particles");
@@ -679,6 +680,7 @@ int Pool::run_substeps(uint32_t substeps) {
 }
 
 int Pool::step(uint32_t substeps) {
+    const Scratch lock(scratch_);
     if (substeps == 0) return fail(LF_ERR_INVALID, "step: zero substeps");
     bool any = false;
     for (const auto &s : scenes_)
@@ -718,6 +720,7 @@ int Pool::to_id_order(uint32_t id) {
 }
 
 int Pool::upload(uint32_t id, uint32_t first, uint32_t count, const float *pos, const float *vel, const float *acc) {
+    const Scratch lock(scratch_);
     const SceneRec *s = scene(id);
     if (!s) return fail(LF_ERR_INVALID, "upload: no scene %u", id);
     if (!pos && count) return fail(LF_ERR_INVALID, "upload: null positions");
@@ -740,6 +743,7 @@ int Pool::upload(uint32_t id, uint32_t first, uint32_t count, const float *pos, 
 }
 
 int Pool::enqueue_upload(uint32_t id, const float *d_stage, uint32_t count) {
+    const Scratch lock(scratch_);
     const SceneRec *s = scene(id);
     if (!s || count > s->n) return fail(LF_ERR_INVALID, "enqueue_upload: bad scene %u or count", id);
     if (int rc = to_id_order(id)) return rc;
@@ -754,6 +758,7 @@ int Pool::enqueue_export(uint32_t id, float *d_out, uint32_t *d_ids, bool by_id)
 }
 
 int Pool::download(uint32_t id, int order, float *pos, float *col, float *vel, float *acc, uint32_t *ids) {
+    const Scratch lock(scratch_);
     const SceneRec *s = scene(id);
     if (!s) return fail(LF_ERR_INVALID, "download: no scene %u", id);
     if (order != LF_ORDER_CELL && order != LF_ORDER_ID) return fail(LF_ERR_INVALID, "download: bad order %d", order);
@@ -968,6 +973,7 @@ int Pool::get_field(uint32_t id, int field, void *dst, size_t bytes) {
 }
 
 int Pool::neighbours(uint32_t id, uint32_t *counts, uint32_t *list, uint64_t cap, uint64_t *total) {
+    const Scratch lock(scratch_);
     const SceneRec *s = scene(id);
     if (!s || !counts) return fail(LF_ERR_INVALID, "neighbours: bad scene or null counts");
     if (!s->active) return fail(LF_ERR_STATE, "neighbours: scene %u is not active", id);
@@ -1113,6 +1119,7 @@ int Pool::set_tuning(const Tuning &t) {
 // scene's step count and order flag) is restored afterwards, so tuning
 // leaves the trajectories untouched.
 int Pool::autotune(uint32_t reps, double ms_out[4][3]) {
+    const Scratch lock(scratch_);
     if (reps == 0) return fail(LF_ERR_INVALID, "autotune: zero reps");
     bool any = false;
     for (const auto &s : scenes_) any |= s.live && s.active && s.dt > 0.0f;
