@@ -167,6 +167,9 @@ int lf_neighbours(lf_scene *s, uint32_t *counts, uint32_t *list, uint64_t cap, u
  * arrays hold 16 elements. */
 int lf_debug_flat_table(const uint64_t masks[9], const uint32_t first_slot[9], uint32_t *entry_mask,
                         uint32_t *entry_base, uint32_t *count);
+/* Test hook: lanes per particle (1 or 4) that the neighbour passes of the
+ * next step take. */
+int lf_debug_lanes(lf_scene *s, int *lanes);
 /* Test hooks for the allocation-failure paths (no counterpart in the
  * reference): after lf_debug_fail_alloc(k) the library's (k+1)-th device
  * allocation from now fails with LF_ERR_ALLOC (k < 0: none fails);
@@ -246,14 +249,17 @@ int lf_export_wait(lf_scene *s);
  *      derived from the largest cell occupancy every substep,
  *      fluidsystem.cu:319-323) ------------------------------------------- */
 /* Workgroup sizes of the density, normals, forces and XSPH passes, each 128,
- * 256 or 512 (default 256); steps of few particles take four lanes per
- * particle in workgroups of 256 whatever is set.  Results do not depend on
- * them. */
+ * 256 or 512 (default 256), and their walk modes (lf_set_walks) shape kernels
+ * with one lane per particle.  While all of them are the default ones, steps
+ * of few particles take four lanes per particle instead, which is faster
+ * there; any other setting is taken as it is, at every size.  Results do not
+ * depend on them. */
 int lf_set_tuning(lf_scene *s, const int block_sizes[4]);
 int lf_get_tuning(const lf_scene *s, int block_sizes[4]);
 /* Walk modes of the normals, forces and XSPH passes: 1 walks the density
- * pass's neighbour masks as one flattened stream of set bits, 0 walks them row by row, 2 flattens
- * only the waves in which a row holds more than 32 slots.  Default {1, 1, 2}
+ * pass's neighbour masks as one flattened stream of set bits, 0 walks them
+ * row by row, 2 flattens only the waves in which a row holds more than 32
+ * slots.  Default {1, 1, 2}
  * (measured fastest: the force walk's arithmetic-heavy steps gain from the
  * flattened stream everywhere, the XSPH walk's gather-heavy ones only where
  * rows are long); lf_autotune picks per pass.  Results do not depend on
@@ -262,7 +268,9 @@ int lf_set_walks(lf_scene *s, const int flat[3]);
 int lf_get_walks(const lf_scene *s, int flat[3]);
 /* Times each block size on the scene's current state (`reps` substeps each,
  * state restored) and keeps the fastest per pass; then, at those block
- * sizes, the three walk modes, keeping the fastest per pass.  ms (may be NULL)
+ * sizes, the three walk modes, keeping the fastest per pass.  All of these
+ * take one lane per particle; steps that would take four by default are timed
+ * that way too, and keep four unless they took longer.  ms (may be NULL)
  * receives the 12 block-size averages: pass-major, block sizes 128, 256, 512.
  * Needs one lf_step first (the substep length). */
 int lf_autotune(lf_scene *s, uint32_t reps, double *ms);
@@ -319,6 +327,7 @@ int lf_batch_get_tuning(const lf_batch *b, int block_sizes[4]);
 int lf_batch_set_walks(lf_batch *b, const int flat[3]);
 int lf_batch_get_walks(const lf_batch *b, int flat[3]);
 int lf_batch_autotune(lf_batch *b, uint32_t reps, double *ms);
+int lf_batch_debug_lanes(lf_batch *b, int *lanes);
 int lf_batch_set_graphs(lf_batch *b, int on);
 int lf_batch_profile_enable(lf_batch *b, int mask);
 int lf_batch_profile_read(lf_batch *b, uint64_t *launches, double *ms);

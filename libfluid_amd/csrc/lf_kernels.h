@@ -29,8 +29,11 @@ struct PoolView {
     uint32_t nlaunch;
     uint8_t *near;
     bool full;  // a scene of the launch has viscosity or surface tension
+    bool one_lane;  // the neighbour passes take one lane per particle whatever the launch's size
 };
 
+// Whether the neighbour passes of a launch take four lanes per particle.
+bool use_quads(const PoolView &pv);
 uint32_t scan_tiles(uint32_t m);
 // Block sizes the neighbour passes are built for (128, 256, 512).
 bool valid_block_size(int bs);

@@ -2455,7 +2455,9 @@ static inline void with_bs(int bs, F &&body) {
 // pairs cost twice as much, 10,000 particles 190 / 90, 65,000 174 / 140 and
 // 308 / 224, 98,000 162 / 157 and 365 / 355, 131,000 521 / 519.
 constexpr uint32_t kQuadSlots = 49152, kQuadSlotsFull = 98304;
-static inline bool use_quads(const PoolView &pv) { return pv.nlaunch <= (pv.full ? kQuadSlotsFull : kQuadSlots); }
+bool use_quads(const PoolView &pv) {
+    return !pv.one_lane && pv.nlaunch <= (pv.full ? kQuadSlotsFull : kQuadSlots);
+}
 
 bool valid_block_size(int bs) { return bs == 128 || bs == 256 || bs == 512; }
 

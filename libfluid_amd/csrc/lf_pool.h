@@ -20,13 +20,20 @@
 
 namespace lf {
 
-// Workgroup sizes of the four neighbour passes (128, 256 or 512 each).
-// Launch shapes: workgroup size per neighbour pass, and whether the normals,
-// forces and XSPH passes walk the neighbour masks as one flattened stream
-// (1) or row by row (0).  Results do not depend on either.
+// Launch shapes: workgroup size per neighbour pass (128, 256 or 512), and
+// whether the normals, forces and XSPH passes walk the neighbour masks as one
+// flattened stream (1), row by row (0) or flattened where rows are long (2).
+// They shape the kernels with one lane per particle; with automatic set,
+// launches of few particles take four lanes instead.  Results do not depend
+// on any of it.
 struct Tuning {
     int density = 256, normals = 256, forces = 256, xsph = 256;
     int flat_normals = 1, flat_forces = 1, flat_xsph = 2;
+    bool automatic = true;
+    bool same_shapes(const Tuning &o) const {
+        return density == o.density && normals == o.normals && forces == o.forces && xsph == o.xsph &&
+               flat_normals == o.flat_normals && flat_forces == o.flat_forces && flat_xsph == o.flat_xsph;
+    }
 };
 
 struct SceneRec {
@@ -110,12 +117,19 @@ class Pool {
     int profile_enable(uint32_t mask);
     int profile_read(uint64_t *launches, double *ms);
     int copy_probe(size_t bytes, int repeats, double *ms);
+    // Shapes other than the default ones are taken as they are set, by
+    // launches of few particles too; the default ones leave those to the
+    // library (Tuning::automatic).
     int set_tuning(const Tuning &t);
     const Tuning &tuning() const { return tune_; }
-    // Times every block size of the neighbour passes on the pool's current
-    // scenes (reps substeps each, state restored afterwards) and keeps the
-    // fastest per pass.  ms[k][b]: average time of pass k (density, normals,
-    // forces, xsph) at block size 128 << b; may be null.
+    // Lanes per particle (1 or 4) the next substep's neighbour passes take.
+    int lanes(int *out);
+    // Times every block size of the neighbour passes (one lane per particle)
+    // on the pool's current scenes (reps substeps each, state restored
+    // afterwards) and keeps the fastest per pass; a pool whose launches take
+    // four lanes keeps doing so unless the four passes took longer that way.
+    // ms[k][b]: average time of pass k (density, normals, forces, xsph) at
+    // block size 128 << b; may be null.
     int autotune(uint32_t reps, double ms[4][3]);
     void set_graphs(bool on);
     // Whether calls of fewer than kGraphRun substeps replay graphs too (the
@@ -158,7 +172,7 @@ class Pool {
     void timed(int kind, Fn &&launch);
     void drop_graph();
     bool any_full() const;
-    PoolView view() const { return PoolView{d_cs_, d_chunk_, nslots_, span_slots_, near_, any_full()}; }
+    PoolView view() const { return PoolView{d_cs_, d_chunk_, nslots_, span_slots_, near_, any_full(), !tune_.automatic}; }
     void set_spans();
 
     // Held by every call that uses the scratch arrays (P1, V1, A1, L1) or the

@@ -1108,16 +1108,26 @@ int Pool::set_tuning(const Tuning &t) {
                         "tuning: walk modes must be 0 (row by row), 1 (flattened) or 2 (flattened in waves with a "
                         "row of more than 32 slots)");
     tune_ = t;
+    tune_.automatic = t.same_shapes(Tuning{});
     drop_graph();
+    return LF_OK;
+}
+
+int Pool::lanes(int *out) {
+    if (!out) return fail(LF_ERR_INVALID, "lanes: null output");
+    const Scratch lock(scratch_);
+    if (int rc = push_tables()) return rc;
+    *out = use_quads(view()) ? 4 : 1;
     return LF_OK;
 }
 
 // Each candidate launch shape runs `reps` substeps from the same saved
 // state, all four neighbour passes timed with events: first the three block
-// sizes (walk modes as set), then, at the fastest block sizes, both walk
-// modes of the normals, forces and XSPH passes.  The state (and every
-// scene's step count and order flag) is restored afterwards, so tuning
-// leaves the trajectories untouched.
+// sizes (walk modes as set), then, at the fastest block sizes, the walk
+// modes of the normals, forces and XSPH passes, all with one lane per
+// particle; then, where the pool's launches would take them, four lanes.  The
+// state (and every scene's step count and order flag) is restored
+// afterwards, so tuning leaves the trajectories untouched.
 int Pool::autotune(uint32_t reps, double ms_out[4][3]) {
     const Scratch lock(scratch_);
     if (reps == 0) return fail(LF_ERR_INVALID, "autotune: zero reps");
@@ -1166,6 +1176,7 @@ int Pool::autotune(uint32_t reps, double ms_out[4][3]) {
     double ms[4][3] = {};
     for (int b = 0; b < 3 && !rc; ++b) {
         Tuning t = before;
+        t.automatic = false;
         t.density = t.normals = t.forces = t.xsph = sizes[b];
         double out[4] = {};
         time_shape(t, out);
@@ -1178,6 +1189,7 @@ int Pool::autotune(uint32_t reps, double ms_out[4][3]) {
             if (ms[k][b] > 0.0 && ms[k][b] < ms[k][best[k]]) best[k] = b;
     }
     Tuning chosen = before;
+    chosen.automatic = false;
     chosen.density = sizes[best[0]];
     chosen.normals = sizes[best[1]];
     chosen.forces = sizes[best[2]];
@@ -1197,6 +1209,15 @@ int Pool::autotune(uint32_t reps, double ms_out[4][3]) {
     chosen.flat_normals = pick(1);
     chosen.flat_forces = pick(2);
     chosen.flat_xsph = pick(3);
+    const double one = ms[0][best[0]] + walk[chosen.flat_normals][1] + walk[chosen.flat_forces][2] +
+                       walk[chosen.flat_xsph][3];
+    chosen.automatic = true;
+    tune_ = chosen;
+    if (!rc && use_quads(view())) {
+        double four[4] = {};
+        time_shape(chosen, four);
+        chosen.automatic = four[0] + four[1] + four[2] + four[3] <= one;
+    }
     prof_mask_ = keep_mask;
     for (auto &r : prof_live_) {  // left over after an error
         ev_pool_.push_back(r.a);

@@ -177,6 +177,16 @@ int lf_debug_flat_table(const uint64_t masks[9], const uint32_t first_slot[9], u
     return LF_OK;
 }
 
+int lf_debug_lanes(lf_scene *s, int *lanes) {
+    if (!s) return fail(LF_ERR_INVALID, "null scene");
+    return s->pool.lanes(lanes);
+}
+
+int lf_batch_debug_lanes(lf_batch *b, int *lanes) {
+    if (!b) return fail(LF_ERR_INVALID, "null batch");
+    return b->pool.lanes(lanes);
+}
+
 int lf_debug_fail_alloc(int64_t nth) {
     lf::debug_fail_alloc(nth);
     return LF_OK;
