@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "lf_abi.h"
 #include "lf_device.h"
 
 namespace lf {
@@ -28,12 +29,14 @@ struct PoolView {
     uint32_t nslots;
     uint32_t nlaunch;
     uint8_t *near;
-    bool full;  // a scene of the launch has viscosity or surface tension
-    bool one_lane;  // the neighbour passes take one lane per particle whatever the launch's size
+    bool quads;  // the neighbour passes take four lanes per particle
 };
 
-// Whether the neighbour passes of a launch take four lanes per particle.
-bool use_quads(const PoolView &pv);
+// How much of the largest launch that takes four lanes per particle `slots`
+// slots of a scene with parameters p make, and whether a launch of nlaunch
+// slots whose active scenes add up to `share` takes them.
+double quad_share(const lf_params &p, uint32_t slots);
+bool takes_quads(double share, uint32_t nlaunch);
 uint32_t scan_tiles(uint32_t m);
 // Block sizes the neighbour passes are built for (128, 256, 512).
 bool valid_block_size(int bs);

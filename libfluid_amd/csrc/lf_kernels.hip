@@ -2447,17 +2447,33 @@ static inline void with_bs(int bs, F &&body) {
     }
 }
 
-// Whether the neighbour passes take four lanes per particle: launches of so
-// few slots that one lane each leaves the chip's 1,024 SIMDs with less than a
-// wave or two.  Measured, a substep with one / four lanes: plain fluid, 32,768
-// particles 58 / 48 us at rest and 80 / 60 in the splash, 65,000 68 / 71 and
-// 91 / 91, 98,000 72 / 84 and 96 / 110; with viscosity or tension, whose
-// pairs cost twice as much, 10,000 particles 190 / 90, 65,000 174 / 140 and
-// 308 / 224, 98,000 162 / 157 and 365 / 355, 131,000 521 / 519.
-constexpr uint32_t kQuadSlots = 49152, kQuadSlotsFull = 98304;
-bool use_quads(const PoolView &pv) {
-    return !pv.one_lane && pv.nlaunch <= (pv.full ? kQuadSlotsFull : kQuadSlots);
+// Which launches take four lanes per particle in the neighbour passes: those
+// whose active scenes hold so few slots that one lane each leaves the chip's
+// 1,024 SIMDs with less than a wave or two.  A slot counts by what its pairs
+// cost: kQuadSlots plain ones fill a launch, or kQuadSlotsFull of scenes with
+// viscosity or tension, or kQuadSlotsLong of those whose stencil rows hold
+// more than 32 slots at rest density.  A substep with one / four lanes, us:
+//   plain, block 49,152 56.4 / 46.5, 61,440 57.3 / 55.8; spray 61,440 58.7 /
+//   57.7; 16 scenes of 4,000 53.1 / 54.2; 65,000 in the splash 91 / 91
+//   full, block 65,536 75.4 / 70.5, 81,920 84.9 / 85.6, 98,304 87.4 / 93.6;
+//   spray (0.4 a cell) 65,536 69.2 / 67.2, 73,728 72.7 / 80.4; 17 scenes of
+//   4,000 80.2 / 81.7, 24 of them 78.9 / 93.5
+//   full with long rows, double dam 81,920 141 / 117 at rest and 377 / 305 in
+//   the splash, 98,304 144 / 129 and 395 / 396; 131,000 521 / 519
+//   mixed, 12 plain scenes of 4,000 and a full one of 500 68.5 / 59.2, 16 and
+//   one 67.7 / 68.5, 16 and 8 of 4,000 78.4 / 92.7
+// Slots of paused scenes only cost their empty workgroups: every other of 24
+// plain scenes of 4,000 paused (98,304 launched) 77.1 / 75.2.  Longer
+// launches take one lane.
+constexpr double kQuadSlots = 61440, kQuadSlotsFull = 65536, kQuadSlotsLong = 98304;
+constexpr uint32_t kQuadLaunch = 98304;
+double quad_share(const lf_params &p, uint32_t slots) {
+    if (p.viscosity == 0.0f && p.surface_tension == 0.0f) return slots / kQuadSlots;
+    const double per_cell =
+        (double)p.rest_density / ((double)p.mass * p.inv_cell[0] * p.inv_cell[1] * p.inv_cell[2]);
+    return slots / (3.0 * per_cell > 32.0 ? kQuadSlotsLong : kQuadSlotsFull);
 }
+bool takes_quads(double share, uint32_t nlaunch) { return nlaunch <= kQuadLaunch && share <= 1.0 + 1e-9; }
 
 bool valid_block_size(int bs) { return bs == 128 || bs == 256 || bs == 512; }
 
@@ -2505,7 +2521,7 @@ void launch_gather(const Launch &L, const PoolView &pv, const uint32_t *slot_src
 void launch_density(const Launch &L, const PoolView &pv, int bs, const float4 *Ps, const float *soa,
                     const uint32_t *start, float4 *D, float4 *Q, float *Pr, RowMasks MS, uint32_t *flags,
                     const uint32_t *moves) {
-    if (use_quads(pv)) {
+    if (pv.quads) {
         LF_GO(L, k_density_quad, pv.nlaunch / kQuadParts, kQuadBlock, L.a, L.b, pv.cs, pv.chunk, pv.nslots, Ps, soa,
               start, D, Q, Pr, MS, flags, moves, pv.near);
         return;
@@ -2519,7 +2535,7 @@ void launch_density(const Launch &L, const PoolView &pv, int bs, const float4 *P
 void launch_normals(const Launch &L, const PoolView &pv, int bs, int flat, bool all, const float4 *Q,
                     const float *soa, const uint32_t *start, RowMasks M, const uint32_t *flags, const uint32_t *moves,
                     float4 *N) {
-    if (use_quads(pv)) {
+    if (pv.quads) {
         LF_GO(L, k_normals_quad, pv.nlaunch / kQuadParts, kQuadBlock, L.a, L.b, pv.cs, pv.chunk, pv.nslots, Q, soa,
               start, M, all ? 1 : 0, flags, moves, pv.near, N);
         return;
@@ -2535,7 +2551,7 @@ void launch_forces(const Launch &L, const PoolView &pv, int bs, int flat, const 
                    const float4 *D, const float4 *N, const float *soa, const uint32_t *start, RowMasks M,
                    float4 *Pout, float4 *Vout, float4 *Aout, float4 *Lout, float4 *Fdbg, uint32_t *flags,
                    const uint32_t *moves) {
-    if (use_quads(pv)) {
+    if (pv.quads) {
         LF_GO(L, k_forces_quad, pv.nlaunch / kQuadParts, kQuadBlock, L.a, L.b, pv.cs, pv.chunk, pv.nslots, Ps, Q, Pr,
               Vs, A, Lw, order, D, N, soa, start, M, Pout, Vout, Aout, Lout, Fdbg, flags, moves, pv.near);
         return;
@@ -2549,7 +2565,7 @@ void launch_forces(const Launch &L, const PoolView &pv, int bs, int flat, const 
 void launch_xsph(const Launch &L, const PoolView &pv, int bs, int flat, const float4 *Ps, const float4 *Pn,
                  const float4 *Vh, const float4 *Lw, const float *soa, const uint32_t *start, RowMasks MS,
                  const uint32_t *flags, const uint32_t *moves, float4 *Vout) {
-    if (use_quads(pv)) {
+    if (pv.quads) {
         LF_GO(L, k_xsph_quad, pv.nlaunch / kQuadParts, kQuadBlock, L.a, L.b, pv.cs, pv.chunk, pv.nslots, Ps, Pn, Vh,
               Lw, soa, start, MS, flags, moves, pv.near, Vout);
         return;

@@ -200,7 +200,7 @@ extern "C" int lf_step_noalloc(const lf_params *p, uint32_t num_particles, float
     const unsigned nb = (num_particles + kBlock - 1) / kBlock;
     hipLaunchKernelGGL(k_na_load, dim3(nb), dim3(kBlock), 0, st, pos_xyz, vel_xyz, acc_xyz, num_particles, b.P0,
                        b.V0, b.A0, b.L0);
-    const PoolView pv{b.cs, b.chunk, slots, slots, b.near, c.has_visc || c.has_tension, false};
+    const PoolView pv{b.cs, b.chunk, slots, slots, b.near, takes_quads(quad_share(*p, slots), slots)};
     const Launch L{st, nullptr, nullptr};
     for (uint32_t k = 0; k < substeps; ++k) {
         // One substep, the pool's sequence (Pool::enqueue_sort, enqueue_substep).

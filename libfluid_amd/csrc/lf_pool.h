@@ -171,8 +171,8 @@ class Pool {
     template <class Fn>
     void timed(int kind, Fn &&launch);
     void drop_graph();
-    bool any_full() const;
-    PoolView view() const { return PoolView{d_cs_, d_chunk_, nslots_, span_slots_, near_, any_full(), !tune_.automatic}; }
+    bool quads() const { return tune_.automatic && takes_quads(quad_share_, span_slots_); }
+    PoolView view() const { return PoolView{d_cs_, d_chunk_, nslots_, span_slots_, near_, quads()}; }
     void set_spans();
 
     // Held by every call that uses the scratch arrays (P1, V1, A1, L1) or the
@@ -190,6 +190,7 @@ class Pool {
     // range, each rounded up to a sixteenth of the pool (so that a captured
     // substep stays valid while scenes come and go below that mark).
     uint32_t span_slots_ = 0, span_buckets_ = 0;
+    double quad_share_ = 0.0;  // of the active scenes' slots, from the same tables
     int debug_ = 0;
     Tuning tune_{};
     bool use_graphs_ = true, short_graphs_ = true;
@@ -243,7 +244,7 @@ class Pool {
     hipGraphExec_t graph_exec_[2][2] = {};
     int parity_ = 0;              // which pairing is current (toggled by advance_state)
     bool graph_normals_ = false;  // the captured substeps have the normals pass
-    bool graph_full_ = false;     // and a scene with viscosity or tension
+    bool graph_quads_ = false;    // and four lanes per particle
     std::vector<std::pair<uint32_t, uint32_t>> graph_paused_;  // and carry these paused scenes' slots
     std::pair<uint32_t, uint32_t> graph_span_{0, 0};         // and cover these spans
 

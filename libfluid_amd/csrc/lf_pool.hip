@@ -310,8 +310,10 @@ int Pool::push_tables() {
 void Pool::set_spans() {
     const uint32_t gs = ((nslots_ / 16 + kChunk - 1) / kChunk) * kChunk, gb = (nbuckets_ + 15) / 16;
     uint64_t es = 0, eb = 0;
+    quad_share_ = 0.0;
     for (const SceneRec &s : scenes_)
         if (s.live && s.active) {
+            quad_share_ += quad_share(s.params, s.nchunks * kChunk);
             es = std::max<uint64_t>(es, s.first + (uint64_t)s.nchunks * kChunk);
             eb = std::max<uint64_t>(eb, s.cell_base + (uint64_t)s.ncells + 1);
         }
@@ -540,12 +542,6 @@ bool Pool::any_separate_normals() const {
     return false;
 }
 
-bool Pool::any_full() const {
-    for (const SceneRec &s : scenes_)
-        if (s.live && s.active && (s.params.viscosity != 0.0f || s.params.surface_tension != 0.0f)) return true;
-    return false;
-}
-
 // Hash, scan, provisional scatter and stable gather of the state positions
 // and velocities (P0, V0) into cell order (P1, V1); ranks_ then holds, per
 // cell-order slot, the particle's state slot (the force pass reads A0 and L0
@@ -638,7 +634,8 @@ int Pool::run_substeps(uint32_t substeps) {
     }
     const std::pair<uint32_t, uint32_t> span{span_slots_, span_buckets_};
     if ((graph_exec_[0][0] || graph_exec_[0][1] || graph_exec_[1][0] || graph_exec_[1][1]) &&
-        (graph_normals_ != any_separate_normals() || graph_full_ != any_full() || graph_paused_ != paused_ranges() || graph_span_ != span))
+        (graph_normals_ != any_separate_normals() || graph_quads_ != quads() || graph_paused_ != paused_ranges() ||
+         graph_span_ != span))
         drop_graph();
     for (uint32_t k = 0; k < substeps;) {
         const int len = substeps - k >= (uint32_t)kGraphRun ? 1 : 0;
@@ -664,7 +661,7 @@ int Pool::run_substeps(uint32_t substeps) {
             }
             graph_[len][parity_] = g;
             graph_normals_ = any_separate_normals();
-            graph_full_ = any_full();
+            graph_quads_ = quads();
             graph_paused_ = paused_ranges();
             graph_span_ = span;
         }
@@ -1117,7 +1114,7 @@ int Pool::lanes(int *out) {
     if (!out) return fail(LF_ERR_INVALID, "lanes: null output");
     const Scratch lock(scratch_);
     if (int rc = push_tables()) return rc;
-    *out = use_quads(view()) ? 4 : 1;
+    *out = quads() ? 4 : 1;
     return LF_OK;
 }
 
@@ -1213,7 +1210,7 @@ int Pool::autotune(uint32_t reps, double ms_out[4][3]) {
                        walk[chosen.flat_xsph][3];
     chosen.automatic = true;
     tune_ = chosen;
-    if (!rc && use_quads(view())) {
+    if (!rc && quads()) {
         double four[4] = {};
         time_shape(chosen, four);
         chosen.automatic = four[0] + four[1] + four[2] + four[3] <= one;
