@@ -170,6 +170,8 @@ int lf_debug_flat_table(const uint64_t masks[9], const uint32_t first_slot[9], u
 /* Test hook: lanes per particle (1 or 4) that the neighbour passes of the
  * next step take. */
 int lf_debug_lanes(lf_scene *s, int *lanes);
+/* Test hook: substep graphs the library has captured so far (lf_set_graphs). */
+int lf_debug_captures(int64_t *count);
 /* Test hooks for the allocation-failure paths (no counterpart in the
  * reference): after lf_debug_fail_alloc(k) the library's (k+1)-th device
  * allocation from now fails with LF_ERR_ALLOC (k < 0: none fails);
@@ -274,9 +276,12 @@ int lf_get_walks(const lf_scene *s, int flat[3]);
  * receives the 12 block-size averages: pass-major, block sizes 128, 256, 512.
  * Needs one lf_step first (the substep length). */
 int lf_autotune(lf_scene *s, uint32_t reps, double *ms);
-/* On (default): lf_step replays one captured hipGraph per substep; off: every
- * kernel is launched individually.  Profiling (lf_profile_enable) always
- * launches individually.  Results are the same either way. */
+/* On (default): lf_step replays captured hipGraphs, of eight substeps and of
+ * one, each captured when it is needed a second time since the parameters,
+ * launch shapes or active scenes changed (before that its kernels are launched
+ * individually); off: every kernel is launched individually.  Profiling
+ * (lf_profile_enable) always launches individually.  Results are the same
+ * either way. */
 int lf_set_graphs(lf_scene *s, int on);
 
 /* ---- batches of independent scenes ------------------------------------

@@ -194,6 +194,7 @@ def _load():
         "lf_server_get_stats": (C.c_int, [C.c_void_p, P(LfServerStats)]),
         "lf_debug_flat_table": (C.c_int, [P(C.c_uint64), u32p, u32p, u32p, u32p]),
         "lf_debug_lanes": (C.c_int, [C.c_void_p, P(C.c_int)]),
+        "lf_debug_captures": (C.c_int, [P(C.c_int64)]),
         "lf_batch_debug_lanes": (C.c_int, [C.c_void_p, P(C.c_int)]),
         "lf_debug_fail_alloc": (C.c_int, [C.c_int64]),
         "lf_debug_live_allocs": (C.c_int, [P(C.c_int64)]),
@@ -225,7 +226,7 @@ EXPORTED = (
     "lf_checkpoint_save lf_checkpoint_load lf_setup_jittered_lattice lf_setup_fluid_block lf_export_geo_async "
     "lf_export_wait lf_batch_checkpoint_save lf_batch_checkpoint_load lf_batch_setup_jittered_lattice "
     "lf_batch_setup_fluid_block lf_batch_export_geo_async lf_batch_export_wait "
-    "lf_debug_lanes lf_batch_debug_lanes lf_debug_flat_table lf_debug_fail_alloc lf_debug_live_allocs lf_step_noalloc"
+    "lf_debug_lanes lf_debug_captures lf_batch_debug_lanes lf_debug_flat_table lf_debug_fail_alloc lf_debug_live_allocs lf_step_noalloc"
 ).split()
 
 

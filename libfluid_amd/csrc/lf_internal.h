@@ -23,6 +23,7 @@ int dev_alloc(void **p, size_t bytes);
 void dev_free_raw(void *p);
 void debug_fail_alloc(int64_t nth);  // nth < 0: never
 int64_t debug_live_allocs();
+int64_t debug_captures();            // substep graphs captured so far (lf_debug_captures)
 template <class T>
 void dev_free(T *&p) {
     if (p) dev_free_raw((void *)p);

@@ -234,19 +234,27 @@ class Pool {
     char *stage_[kStages] = {};
     hipEvent_t stage_ev_[kStages] = {};
 
-    // captured substep, one per pairing of the state and scratch A/L buffers,
+    // Captured substeps, one per pairing of the state and scratch A/L buffers,
     // and the same for runs of kGraphRun substeps ([1]): between two graph
     // launches the device idles for about 6 us (a substep replayed one by one
     // / in runs of 8: 2,000 particles 44.7 / 39.0 us, 131,000 81.1 / 74.8,
-    // 1,048,576 277.9 / 272.2).
+    // 1,048,576 277.9 / 272.2).  What is needed for the first time is launched
+    // kernel by kernel instead, a single substep throughout that call: the
+    // device starts at once, and a program that changes its scene before every
+    // call captures nothing.
     static constexpr int kGraphRun = 8;  // even: a run leaves the buffers as it found them
+    struct GraphKey {
+        bool normals = false, quads = false;                // the normals pass; four lanes per particle
+        std::pair<uint32_t, uint32_t> span{0, 0};           // slots and buckets covered
+        std::vector<std::pair<uint32_t, uint32_t>> paused;  // paused scenes' slots, carried across
+        bool operator==(const GraphKey &) const = default;
+    };
     hipGraph_t graph_[2][2] = {};
     hipGraphExec_t graph_exec_[2][2] = {};
-    int parity_ = 0;              // which pairing is current (toggled by advance_state)
-    bool graph_normals_ = false;  // the captured substeps have the normals pass
-    bool graph_quads_ = false;    // and four lanes per particle
-    std::vector<std::pair<uint32_t, uint32_t>> graph_paused_;  // and carry these paused scenes' slots
-    std::pair<uint32_t, uint32_t> graph_span_{0, 0};         // and cover these spans
+    uint64_t graph_seen_[2][2] = {};  // the call that needed it first (0: none yet)
+    uint64_t graph_call_ = 0;
+    GraphKey graph_key_;
+    int parity_ = 0;  // which pairing is current (toggled by advance_state)
 
     Exporter *exporter_ = nullptr;
 

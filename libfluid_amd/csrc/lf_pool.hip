@@ -30,6 +30,7 @@ namespace {
 
 std::atomic<int64_t> g_live_allocs{0};  // device allocations the library holds
 std::atomic<int64_t> g_fail_at{-1};     // allocations to go before one fails (-1: never)
+std::atomic<int64_t> g_captures{0};     // substep graphs captured so far
 
 }  // namespace
 
@@ -50,6 +51,7 @@ int dev_alloc(void **p, size_t bytes) {
 
 void debug_fail_alloc(int64_t nth) { g_fail_at.store(nth < 0 ? -1 : nth); }
 int64_t debug_live_allocs() { return g_live_allocs.load(); }
+int64_t debug_captures() { return g_captures.load(); }
 
 void dev_free_raw(void *p) {
     if (!p) return;
@@ -615,6 +617,7 @@ void Pool::drop_graph() {
             if (graph_[l][p]) (void)hipGraphDestroy(graph_[l][p]);
             graph_exec_[l][p] = nullptr;
             graph_[l][p] = nullptr;
+            graph_seen_[l][p] = 0;
         }
 }
 
@@ -632,21 +635,32 @@ int Pool::run_substeps(uint32_t substeps) {
         }
         return check_launch("step");
     }
-    const std::pair<uint32_t, uint32_t> span{span_slots_, span_buckets_};
-    if ((graph_exec_[0][0] || graph_exec_[0][1] || graph_exec_[1][0] || graph_exec_[1][1]) &&
-        (graph_normals_ != any_separate_normals() || graph_quads_ != quads() || graph_paused_ != paused_ranges() ||
-         graph_span_ != span))
+    // What a captured substep depends on; tables that change without it need
+    // no new capture, as the substeps read them from device memory.
+    GraphKey key{any_separate_normals(), quads(), {span_slots_, span_buckets_}, paused_ranges()};
+    if (!(graph_key_ == key)) {
         drop_graph();
+        graph_key_ = std::move(key);
+    }
+    ++graph_call_;
     for (uint32_t k = 0; k < substeps;) {
         const int len = substeps - k >= (uint32_t)kGraphRun ? 1 : 0;
+        const uint32_t count = len ? (uint32_t)kGraphRun : 1u;
         hipGraphExec_t &ge = graph_exec_[len][parity_];
+        uint64_t &seen = graph_seen_[len][parity_];
+        if (!ge && (seen == 0 || (!len && seen == graph_call_))) {
+            if (!seen) seen = graph_call_;
+            for (uint32_t q = 0; q < count; ++q) {
+                enqueue_substep();
+                advance_state();
+            }
+            if (int rc = check_launch("step")) return rc;
+            k += count;
+            continue;
+        }
         if (!ge) {
-            // One substep, or kGraphRun of them, captured once per pairing of
-            // the state and scratch A/L buffers; the scene table they read
-            // lives in device memory, so later table changes need no new
-            // capture.
             LF_HIP(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
-            for (int q = 0; q < (len ? kGraphRun : 1); ++q) {
+            for (uint32_t q = 0; q < count; ++q) {
                 enqueue_substep();
                 if (len) advance_state();  // an even number of times
             }
@@ -660,18 +674,11 @@ int Pool::run_substeps(uint32_t substeps) {
                 return fail(LF_ERR_HIP, "step: graph instantiation failed: %s", hipGetErrorString(e));
             }
             graph_[len][parity_] = g;
-            graph_normals_ = any_separate_normals();
-            graph_quads_ = quads();
-            graph_paused_ = paused_ranges();
-            graph_span_ = span;
+            g_captures.fetch_add(1);
         }
         LF_HIP(hipGraphLaunch(ge, stream_));
-        if (len) {
-            k += kGraphRun;
-        } else {
-            advance_state();
-            ++k;
-        }
+        if (!len) advance_state();
+        k += count;
     }
     return LF_OK;
 }

@@ -192,6 +192,12 @@ int lf_debug_fail_alloc(int64_t nth) {
     return LF_OK;
 }
 
+int lf_debug_captures(int64_t *count) {
+    if (!count) return fail(LF_ERR_INVALID, "null count");
+    *count = lf::debug_captures();
+    return LF_OK;
+}
+
 int lf_debug_live_allocs(int64_t *count) {
     if (!count) return fail(LF_ERR_INVALID, "null count");
     *count = lf::debug_live_allocs();

@@ -1,0 +1,58 @@
+"""GPU: when substeps are captured into graphs: only what is needed a second time
+with the same parameters, launch shapes and active scenes."""
+import ctypes as C
+
+import pytest
+
+from libfluid_amd import _lib as L
+from libfluid_amd import configs
+
+pytestmark = pytest.mark.gpu
+
+
+def captures():
+    k = C.c_int64(0)
+    L.check(L.lib.lf_debug_captures(C.byref(k)), "lf_debug_captures")
+    return k.value
+
+
+def test_nothing_is_captured_before_its_second_use(gpu):
+    """A scene whose parameters change before every call captures no graph;
+    one that does not captures each run and single substep once, when it is
+    needed again."""
+    cfg = configs.scaled_c1(12, 10, 8)
+    with gpu.Scene(cfg.params, cfg.n) as sc:
+        sc.upload(cfg.pos)
+        at = captures()
+        p = L.LfParams.from_buffer_copy(cfg.params)
+        for k in (10, 8, 1, 15, 7):
+            p.gravity[0] += 0.25
+            sc.set_params(p)
+            sc.step(1e-4 * k, k)
+            assert captures() == at, k
+        sc.step(1e-4 * 8, 8)   # after 7 single ones: the other pairing's first run
+        assert captures() == at
+        sc.step(1e-4 * 24, 24)
+        assert captures() == at + 1
+        sc.step(1e-4 * 2, 2)   # singles of both pairings, for the second call
+        assert captures() == at + 3
+        for k in (2, 8, 10):
+            sc.step(1e-4 * k, k)
+        assert captures() == at + 3
+    with gpu.Scene(cfg.params, cfg.n) as sc:
+        sc.upload(cfg.pos)
+        sc.step(1e-4 * 16, 16)
+        assert captures() == at + 4
+
+
+def test_paused_and_resumed_scenes_capture_nothing(gpu):
+    scenes = [configs.block_scene(n, (1.6, 1.7, 1.8), (0.1, -1.0, 0.3), seed=n) for n in (700, 1500)]
+    with gpu.Batch(2 * 4096, sum(c.params.ncells + 1 for c in scenes), 2) as b:
+        ids = [b.add(c.params, c.n, 1e-4) for c in scenes]
+        for i, c in zip(ids, scenes):
+            b.upload(i, c.pos)
+        at = captures()
+        for k in range(6):
+            b.set_active(ids[1], k % 2 == 0)
+            b.step(9)
+        assert captures() == at
