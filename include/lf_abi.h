@@ -375,9 +375,10 @@ int lf_server_submit(lf_server *s, const lf_params *p, uint32_t num_particles, c
 /* One serving iteration; *finished = jobs whose results arrived during it. */
 int lf_server_tick(lf_server *s, uint32_t *finished);
 /* run_ahead: batched steps a tick may queue ahead of the device (default 2;
- * 0 makes every tick wait for its step and retirements); graphs: allow
- * captured substeps (default on; a tick's single substep is launched kernel by
- * kernel either way, which is faster).  Results do not depend on either. */
+ * 0 makes every tick wait for its step and retirements); graphs: replay
+ * captured substeps in ticks that wait (default on; ticks that run ahead
+ * launch kernel by kernel either way, which is faster there).  Results do not
+ * depend on either. */
 int lf_server_configure(lf_server *s, uint32_t run_ahead, int graphs);
 /* Moves up to cap ids of jobs finished since the last call into jobs[]. */
 int lf_server_take_finished(lf_server *s, uint64_t *jobs, uint32_t cap, uint32_t *count);

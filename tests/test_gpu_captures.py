@@ -2,10 +2,12 @@
 with the same parameters, launch shapes and active scenes."""
 import ctypes as C
 
+import numpy as np
 import pytest
 
 from libfluid_amd import _lib as L
 from libfluid_amd import configs
+from libfluid_amd.serve import Server
 
 pytestmark = pytest.mark.gpu
 
@@ -56,3 +58,22 @@ def test_paused_and_resumed_scenes_capture_nothing(gpu):
             b.set_active(ids[1], k % 2 == 0)
             b.step(9)
         assert captures() == at
+
+
+@pytest.mark.parametrize("run_ahead,graphs,want", [(0, True, 2), (0, False, 0), (2, True, 0), (2, False, 0)])
+def test_server_ticks_replay_graphs_where_they_wait(gpu, run_ahead, graphs, want):
+    cfg = configs.scaled_c1(12, 10, 8)
+    with Server(2048, cfg.params.ncells + 1, 2) as srv:
+        srv.configure(run_ahead, graphs)
+        at = captures()
+        job = srv.submit(cfg.params, cfg.pos, None, cfg.dt, 9)
+        while not srv.tick():
+            pass
+        assert captures() == at + want
+        got = srv.result(job)
+    with gpu.Scene(cfg.params, cfg.n) as sc:
+        sc.upload(cfg.pos)
+        sc.run(cfg.dt, 9)
+        ref = sc.download(L.LF_ORDER_ID)
+    for k in ("pos", "vel", "acc"):
+        assert np.array_equal(got[k], ref[k]), k
