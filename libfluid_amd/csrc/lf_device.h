@@ -174,8 +174,9 @@ __device__ __forceinline__ bool flag_set(uint32_t word, uint32_t byte) { return 
 // (1 + s) h with s = q / 4096 between kSkinMin and kSkinMax.  A particle
 // that still moves farther than skin_move_limit (a wall projection of a
 // particle that started outside, or a move above the kSkinMax skin) sets
-// the scene's far-move flag and the XSPH pass scans: the result is the same
-// either way, only the speed differs.
+// the scene's far-move flag, and the XSPH pass tests every slot of its rows
+// again on the integrated positions instead of taking the masks: the result
+// is the same either way, only the speed differs.
 constexpr uint32_t kSkinQMax = 512u;  // s = 1/8: above kSkinMax
 constexpr uint32_t kMoveSlots = 16u, kMoveStride = 32u;  // words per scene: kMoveSlots * kMoveStride
 __device__ __forceinline__ uint32_t *move_slot(uint32_t *moves, uint32_t scene, uint32_t k) {

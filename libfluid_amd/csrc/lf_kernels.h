@@ -44,8 +44,9 @@ bool valid_block_size(int bs);
 // Also clears the count of large-bucket segments (nsegs).
 void launch_hash(const Launch &L, const PoolView &pv, const float4 *P, uint32_t *keys, uint32_t *ranks,
                  uint32_t *counts, uint32_t *flags, uint32_t *moves, uint32_t *nsegs);
-// Exclusive scan of counts[0, m) into start[0, m] (start[m] = total), which
-// also clears the counts; bsum holds scan_tiles(m) + 1 words.
+// Exclusive scan of counts[0, m) into start[0, m] (start[m] = total); bsum
+// holds scan_tiles(m) + 1 words.  The counts are cleared by this scan or, where
+// one launch does it, by the scatter that follows.
 void launch_scan(const Launch &L, uint32_t *counts, uint32_t m, uint32_t *bsum, uint32_t *start);
 // Provisional slots by atomic rank; then every bucket of more than
 // kRankDirectMax particles is sorted by id in place (its segment listed in

@@ -23,10 +23,11 @@
 // The density pass tests every candidate of the clipped 27-cell stencil (nine
 // contiguous x-row slot ranges) and records, per row, a 32/64-bit mask of the
 // slots within a skin radius h_s >= h (of its first 96 slots; RowMasks).
-// The normals, forces and XSPH passes walk those masks over packed neighbour data (XSPH when the substep's
-// largest move proves them complete) and re-test each pair; set bits are
-// visited in slot order, so every pass sums the same neighbours in the same
-// order as a full stencil scan, bit for bit.
+// The normals, forces and XSPH passes walk those masks over packed neighbour
+// data (XSPH when the substep's largest move proves them complete; otherwise
+// it makes such masks from the moved positions) and re-test each pair; set
+// bits are visited in slot order, so every pass sums the same neighbours in
+// the same order as a full stencil scan, bit for bit.
 //
 // SPH here is a gather-bound stencil, not a dense contraction: the kernels
 // are VALU/L1 work over the stencil walk and never use MFMA.
@@ -207,8 +208,9 @@ __global__ __launch_bounds__(kBlock) void k_scan_down(uint32_t *__restrict__ cou
 // launch: each workgroup adds up the counts of every tile before its own
 // (eight 16-byte loads in flight per thread) instead of waiting for a first
 // launch to do so: a replayed substep of 2,000 particles 46.0 -> 44.4 us, of
-// 60,000 (64,000 buckets) 64.5 -> 63.9; at 20 tiles the two ways are even.  The counts are cleared by k_scatter, as other workgroups
-// still read them here.
+// 60,000 (64,000 buckets) 64.5 -> 63.9; at 20 tiles the two ways are even.
+// The counts are cleared by k_scatter, as other workgroups still read them
+// here.
 constexpr int kScanOneThreads = 1024;
 constexpr uint32_t kScanOneTile = 4u * kScanOneThreads, kScanOneTiles = 16u;
 __global__ __launch_bounds__(kScanOneThreads) void k_scan_one(const uint32_t *__restrict__ counts, uint32_t m,
@@ -887,8 +889,10 @@ __device__ __forceinline__ bool walk_flat(uint2 *__restrict__ tab, const RowSour
     return WL != 0;
 }
 
-// Walk over the neighbour slots of lane i: with flat set, the flattened walk
-// when masks are in use and every lane's rows fit it, else walk_masks.  The
+// Walk over the neighbour slots of lane i: with flat set and masks in use the
+// flattened walk, unless it declines (walk_flat: a near-isolated wave whose
+// rows need more than one table or whose particles moved far, or, in mode 2,
+// a wave without rows of more than 32 slots); else walk_masks.  The
 // choice is wave-uniform and does not change the result.  A callback is
 // inlined into both walks (and every block size), and an implicit
 // multiply-add contraction may differ between those copies: the callbacks
@@ -1611,10 +1615,11 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(BS >= 512 ? 
 // lanes (density / forces / XSPH of the 32,768-particle dam break in its
 // splash: 20.2 / 19.2 / 15.7 us with one lane, 13.5 / 13.0 / 9.8 with four;
 // density / normals / forces / XSPH of the driver's default scene: 28 / 41 /
-// 72 / 90 and 14 / 15 / 25 / 30).  Sums stay in slot order, so every bit is that of the one-lane
-// kernels: each lane computes the terms of its candidates, then the quad's
-// lanes take turns adding theirs to the running sums, the result of each turn
-// broadcast to the quad (DPP).
+// 72 / 90 and 14 / 15 / 25 / 30; quad_share says which launches).  Sums stay
+// in slot order, so every bit is that of the one-lane kernels: each lane
+// computes the terms of its candidates, then the quad's lanes take turns
+// adding theirs to the running sums, the result of each turn broadcast to the
+// quad (DPP).
 constexpr int kQuadBlock = 256;                 // 64 particles per workgroup
 constexpr uint32_t kQuadParts = kQuadBlock / 4;
 constexpr uint32_t kQuadList = 128;             // neighbour slots of a particle listed at a time

@@ -247,7 +247,7 @@ int Pool::init(uint32_t slot_cap, uint32_t bucket_cap, uint32_t scene_cap) {
         if (e != hipSuccess) rc = fail(LF_ERR_ALLOC, "pool: pinned staging: %s", hipGetErrorString(e));
     }
     if (!rc) {
-        // Counts start at zero; afterwards every scan clears them.
+        // Counts start at zero; afterwards every scan or scatter clears them.
         e = hipMemsetAsync(counts_, 0, sizeof(uint32_t) * nbuckets_, stream_);
         if (e == hipSuccess) e = hipMemsetAsync(start_, 0, sizeof(uint32_t) * (nbuckets_ + 1), stream_);
         if (e == hipSuccess) e = hipMemsetAsync(nsegs_, 0, sizeof(uint32_t), stream_);

@@ -198,7 +198,9 @@ class Scene:
 
     # -- launch shapes ------------------------------------------------------
     def set_tuning(self, block_sizes) -> None:
-        """Workgroup sizes of the density, normals, forces and XSPH passes."""
+        """Workgroup sizes of the density, normals, forces and XSPH passes;
+        with the default sizes and walk modes, steps of few particles take
+        four lanes per particle instead."""
         bs = (C.c_int * 4)(*[int(b) for b in block_sizes])
         check(lib.lf_set_tuning(self._h, bs), "lf_set_tuning")
 
