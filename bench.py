@@ -129,7 +129,7 @@ def batched(args) -> dict:
     b.step(W)
     b.sync()
     tune_ms = b.autotune(3)
-    b.step(1)  # capture the graph with the tuned shapes
+    b.step(1)  # the first step with the tuned shapes
     b.sync()
     t0 = time.perf_counter()
     b.step(K)
@@ -243,8 +243,8 @@ def served(args) -> dict:
     lat = np.array(list(r["latency_ms"].values()))
     # The same jobs alone, on a sample of 32: each stepped for its full step
     # count (the same work it does in the server), one after another, with
-    # graph replay; timed from the first substep (after one warm-up substep
-    # that captures the graph) to the last.
+    # graph replay; timed from the first substep (after one warm-up substep) to
+    # the last.
     rng = np.random.Generator(np.random.PCG64(6))
     sample = rng.choice(len(jobs), size=min(32, len(jobs)), replace=False)
     ps, ts = 0, 0.0
@@ -574,8 +574,9 @@ def main():
 
     sc.close()
 
-    # The same K steps from the same state, unprofiled: each substep replays
-    # the captured hipGraph (the first one captures it, inside the timing).
+    # The same K steps from the same state, unprofiled: each substep replays a
+    # captured hipGraph (the first two launch kernel by kernel and the next two
+    # capture one each, inside the timing).
     sc = lf.Scene.checkpoint_load(ck_path)
     os.unlink(ck_path)
     if args.scan:
