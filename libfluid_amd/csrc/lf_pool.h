@@ -108,6 +108,8 @@ class Pool {
 
     // Enqueues `substeps` substeps of every active scene and returns.
     int step(uint32_t substeps);
+    // The same after set_dt(id, dt), in one turn.
+    int step_scene(uint32_t id, float dt, uint32_t substeps);
     int sync();
 
     // Inspection of the last substep, tuning, timing.

@@ -483,6 +483,7 @@ int Pool::set_params(uint32_t id, const lf_params &p) {
 }
 
 int Pool::set_dt(uint32_t id, float dt) {
+    const Scratch lock(scratch_);
     if (!scene(id)) return fail(LF_ERR_INVALID, "set_dt: no scene %u", id);
     if (!(std::isfinite(dt) && dt > 0.0f)) return fail(LF_ERR_INVALID, "set_dt: dt must be positive and finite");
     if (scenes_[id].dt != dt) {
@@ -702,6 +703,12 @@ int Pool::step(uint32_t substeps) {
         }
     }
     return LF_OK;
+}
+
+int Pool::step_scene(uint32_t id, float dt, uint32_t substeps) {
+    const Scratch lock(scratch_);
+    if (int rc = set_dt(id, dt)) return rc;
+    return step(substeps);
 }
 
 int Pool::sync() {

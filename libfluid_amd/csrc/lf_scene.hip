@@ -136,8 +136,7 @@ int lf_step(lf_scene *s, float dt, uint32_t substeps) {
     // part_dt = full_dt / substeps (fluidsystem.cu:295); exactly `substeps`
     // substeps run (the reference's float-accumulated loop, :301, can run one
     // fewer).
-    if (int rc = s->pool.set_dt(s->id, dt / float(substeps))) return rc;
-    return s->pool.step(substeps);
+    return s->pool.step_scene(s->id, dt / float(substeps), substeps);
 }
 
 int lf_sync(lf_scene *s) {

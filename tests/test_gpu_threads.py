@@ -87,3 +87,22 @@ def test_downloads_beside_steps(gpu, n):
         got = sc.download()
         for k in STATE:
             assert np.array_equal(got[k], seen[-1][k]), k
+
+
+def test_steps_of_two_threads_keep_their_lengths(gpu):
+    """A lone particle stepped by two threads with different step lengths falls
+    for the sum of them: each call's length belongs to its own substeps."""
+    p = configs.scaled_c1(2, 2, 2).params
+    k, d1, d2 = 300, 1e-4, 3e-4
+    with gpu.Scene(p, 1) as sc:
+        sc.upload(np.array([[0.5, 0.45, 0.25]], np.float32))
+
+        def body(dt):
+            for _ in range(k):
+                sc.step(dt, 1)
+
+        run(lambda: body(d1), lambda: body(d2))
+        v = sc.download()["vel"][0]
+    # one step's half is integrated with the acceleration before it (zero at first)
+    assert abs(float(v[1]) + 9.8 * k * (d1 + d2)) <= 0.5 * 9.8 * d2 + 1e-4
+    assert v[0] == 0.0 and v[2] == 0.0
